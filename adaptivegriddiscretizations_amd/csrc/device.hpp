@@ -921,27 +921,35 @@ template <int N> struct MergeNet {
   }
 };
 
-template <class S, int N> __device__ inline void sort_pairs(S (&v)[N], S (&w)[N]) {
+// CEX::swap(vi, wi, vj, wj) orders two pairs.
+template <class CEX, class S, int N> __device__ inline void sort_pairs_by(S (&v)[N], S (&w)[N]) {
   if constexpr (N == 1) {
     // nothing to sort
   } else if constexpr (N == 2) {
-    cex(v[0], w[0], v[1], w[1]);
+    CEX::swap(v[0], w[0], v[1], w[1]);
   } else if constexpr (N == 3) {
-    cex(v[1], w[1], v[2], w[2]); cex(v[0], w[0], v[2], w[2]); cex(v[0], w[0], v[1], w[1]);
+    CEX::swap(v[1], w[1], v[2], w[2]); CEX::swap(v[0], w[0], v[2], w[2]); CEX::swap(v[0], w[0], v[1], w[1]);
   } else if constexpr (N == 6) {
-    cex(v[1], w[1], v[2], w[2]); cex(v[4], w[4], v[5], w[5]);
-    cex(v[0], w[0], v[2], w[2]); cex(v[3], w[3], v[5], w[5]);
-    cex(v[0], w[0], v[1], w[1]); cex(v[3], w[3], v[4], w[4]); cex(v[2], w[2], v[5], w[5]);
-    cex(v[0], w[0], v[3], w[3]); cex(v[1], w[1], v[4], w[4]);
-    cex(v[2], w[2], v[4], w[4]); cex(v[1], w[1], v[3], w[3]);
-    cex(v[2], w[2], v[3], w[3]);
+    CEX::swap(v[1], w[1], v[2], w[2]); CEX::swap(v[4], w[4], v[5], w[5]);
+    CEX::swap(v[0], w[0], v[2], w[2]); CEX::swap(v[3], w[3], v[5], w[5]);
+    CEX::swap(v[0], w[0], v[1], w[1]); CEX::swap(v[3], w[3], v[4], w[4]); CEX::swap(v[2], w[2], v[5], w[5]);
+    CEX::swap(v[0], w[0], v[3], w[3]); CEX::swap(v[1], w[1], v[4], w[4]);
+    CEX::swap(v[2], w[2], v[4], w[4]); CEX::swap(v[1], w[1], v[3], w[3]);
+    CEX::swap(v[2], w[2], v[3], w[3]);
   } else {
     // other lengths (the curvature models' 7 and 30)
     constexpr MergeNet<N> net{};
     constexpr int count = net.n;
 #pragma unroll
-    for (int c = 0; c < count; ++c) cex(v[net.a[c]], w[net.a[c]], v[net.b[c]], w[net.b[c]]);
+    for (int c = 0; c < count; ++c) CEX::swap(v[net.a[c]], w[net.a[c]], v[net.b[c]], w[net.b[c]]);
   }
+}
+
+struct CexTies {
+  template <class S> __device__ static inline void swap(S& vi, S& wi, S& vj, S& wj) { cex(vi, wi, vj, wj); }
+};
+template <class S, int N> __device__ inline void sort_pairs(S (&v)[N], S (&w)[N]) {
+  sort_pairs_by<CexTies, S, N>(v, w);
 }
 
 // HFM.h:165-195: smallest solution of sum_k w_k (u - v_k)_+^2 = rhs^2 over

@@ -26,6 +26,7 @@
 #include "common.hpp"
 #include "device.hpp"
 #include "eikonal_kernels.hpp"
+#include "region_kernels.hpp"
 #include "worklist.hpp"
 
 static_assert(sizeof(agd_eikonal_desc) == 320, "agd_eikonal_desc layout changed");
@@ -414,6 +415,7 @@ template <class T> static void free_dev(T*& p) {
 void Workspace::release() {
   if (!fixed) {
     free_dev(ftab);
+    free_dev(region);
     free_dev(stamp);
     free_dev(needs);
     free_dev(pending);
@@ -440,8 +442,8 @@ void Workspace::release() {
   ev0 = ev1 = chunk_ev[0] = chunk_ev[1] = nullptr;
   capture_stream = nullptr;
   tile_cap = shard_cap = hist_cap = inst_cap = tinst_cap = 0;
-  ftab = nullptr;
-  ftab_bytes = 0;
+  ftab = region = nullptr;
+  ftab_bytes = region_bytes = 0;
   fixed = false;
 }
 
@@ -451,6 +453,17 @@ int Workspace::ensure_ftab(size_t bytes) {
     free_dev(ftab);
     AGD_HIP_TRY(hipMalloc(&ftab, bytes));
     ftab_bytes = bytes;
+  }
+  return AGD_OK;
+}
+
+int Workspace::ensure_region(size_t bytes) {
+  AGD_REQUIRE(!fixed, "the one-launch solve needs an allocating workspace");
+  if (region_bytes < bytes) {
+    free_dev(region);
+    region_bytes = 0;
+    AGD_HIP_TRY(hipMalloc(&region, bytes));
+    region_bytes = bytes;
   }
   return AGD_OK;
 }
@@ -563,6 +576,144 @@ int blocks_for(int ntiles, int lanes_per_block) {
   return std::max(1, std::min(ntiles, target));
 }
 
+// ------------------------------------------------------------------ one launch
+// The cut of the grid for the one-launch solve: one region per compute unit at
+// most, of 32 boxes at most; false where the grid does not fit.
+static bool region_plan(const agd_eikonal_desc* d, const int* box, int waves, size_t (*need)(int), RegionPlan& p) {
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+    return false;
+  const size_t room = (size_t(160) << 10) - 4096;  // LDS of a compute unit, less the static arrays
+  const int D = d->ndim;
+  p = RegionPlan{};
+  for (int c = 0; c < 3; ++c) {
+    p.shape[c] = c < D ? int32_t(d->shape[c]) : 1;
+    p.ntl[c] = c < D ? int32_t(ceil_div(d->shape[c], D == 2 ? 8 : 4)) : 1;
+    p.so[c] = c < D ? int32_t(ceil_div(d->shape[c], d->shape_i[c])) : 1;
+    if (c < D) {
+      if (d->shape_i[c] & (d->shape_i[c] - 1)) return false;
+      while ((1 << p.ls[c]) < d->shape_i[c]) ++p.ls[c];
+      p.lsum += p.ls[c];
+      if (d->periodic[c]) p.periodic |= 1 << c;
+    }
+  }
+  p.nboxes = 1;
+  for (int c = 0; c < 3; ++c) {
+    p.nbox[c] = int32_t(ceil_div(p.ntl[c], box[c]));
+    p.nboxes *= p.nbox[c];
+  }
+  const int per = int(ceil_div(p.nboxes, cus));  // boxes of a region
+  if (per > 32) return false;
+  p.nregions = int32_t(ceil_div(p.nboxes, per));
+  p.ntot = per * waves;
+  return need(p.ntot) <= room;
+}
+
+// One solve of this kind at a time on a device: its workgroups wait for each
+// other, so two of them could each hold half of the compute units.  A solve
+// that finds another one running takes the pass solver instead.
+static std::mutex g_region_mutex[64];
+
+template <class S> static RegionKernels<S> region_lookup(int model, int d) {
+  switch (model) {
+    case AGD_ISOTROPIC:
+    case AGD_DIAGONAL: return region_plain<S>(model, d);
+    case AGD_RIEMANN:
+    case AGD_RANDER: return region_metric<S>(model, d);
+  }
+  if constexpr (std::is_same<S, float>::value) return region_stored(model, d);
+  return {};
+}
+
+// The one-launch solve.  taken: false if it does not apply or gave up, in
+// which case the values are a supersolution (touched: no longer the initial one).
+template <class S>
+static int region_impl(Workspace& ws, const EikArgs<S>& e, const agd_eikonal_desc* d,
+                       const agd_eikonal_io* io, agd_eikonal_stats* stats, hipStream_t stream, bool& taken,
+                       bool& touched) {
+  taken = touched = false;
+  RegionPlan p;
+  int dev = 0;
+  const RegionKernels<S> rk = region_lookup<S>(d->model, d->ndim);
+  if (!rk.solve || hipGetDevice(&dev) != hipSuccess || dev >= 64 || !region_plan(d, rk.box, rk.waves, rk.lds, p))
+    return AGD_OK;
+  std::unique_lock<std::mutex> lock(g_region_mutex[dev], std::try_to_lock);
+  if (!lock.owns_lock()) return AGD_OK;
+  const int64_t ntiles = int64_t(p.nregions) * p.ntot;
+  auto up = [](size_t b) { return (b + 255) & ~size_t(255); };
+  const size_t b_ctl = up(kRegionCtl * 4), b_rest = up(size_t(p.nregions) * 4),
+               b_done = up(size_t(p.nregions) * kRegionLine * 4), b_marks = up(size_t(ntiles) * 4),
+               b_read = up(size_t(ntiles) * 8), b_zero = b_ctl + b_rest + b_done + b_marks + b_read, b_link = up(size_t(ntiles) * 256),
+               b_blk = size_t(ntiles) * size_t(rk.tile_bytes);
+  int st = ws.ensure(1, 1, 1);
+  if (!st) st = ws.ensure_region(b_zero + b_link + b_blk);
+  if (st) return st;
+  char* base = static_cast<char*>(ws.region);
+  RegionArgs<S> a{};
+  a.p = p;
+  a.u = e.u;
+  a.geom = e.geom;
+  a.sw = e.sw;
+  a.scode = e.scode;
+  a.rhs = e.rhs;
+  a.seeds = e.seeds;
+  a.trigger = io->trigger ? io->trigger : io->seeds;
+  a.wall = e.wall;
+  a.size_tot = e.g.size_tot;
+  for (int k = 0; k < 3; ++k) a.iso_w[k] = e.iso_w[k];
+  // Marks are made from a twentieth of the tolerance on: a tile is visited many
+  // more times than it has passes in the pass solver, and each visit may leave a
+  // change below the tolerance unannounced (isotropic2 512^2: error 4.7e-6 of the
+  // values with the tolerance itself, 1.7e-7 with a twentieth, 1.5e-7 with 0 and
+  // with the pass solver; 0 costs 15 % more visits).
+  a.atol = e.atol * S(0.05);
+  a.rtol = e.rtol * S(0.05);
+  a.activate_all = d->activate_all;
+  a.window = 4.f;
+  a.ctl = reinterpret_cast<uint32_t*>(base);
+  a.rest = reinterpret_cast<uint32_t*>(base + b_ctl);
+  a.done = reinterpret_cast<uint32_t*>(base + b_ctl + b_rest);
+  a.marks = reinterpret_cast<uint32_t*>(base + b_ctl + b_rest + b_done);
+  a.readers = reinterpret_cast<uint64_t*>(base + b_zero - b_read);
+  a.links = reinterpret_cast<int32_t*>(base + b_zero);
+  a.blocks = base + b_zero + b_link;
+  a.start_ticks = 500000;     // 5 ms of the 100 MHz clock
+  a.limit_ticks = 100000000;  // 1 s
+  const size_t lds = rk.lds(p.ntot);
+  AGD_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(rk.solve),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
+  AGD_HIP_TRY(hipEventRecord(ws.ev0, stream));
+  fill_i32(reinterpret_cast<int32_t*>(base), int64_t(b_zero / 4), 0, stream);
+  const unsigned wg = unsigned(ceil_div(ntiles, 4));
+  hipLaunchKernelGGL(rk.setup, dim3(wg), dim3(256), 0, stream, a);
+  hipLaunchKernelGGL(rk.links, dim3(wg), dim3(256), 0, stream, p, a.readers, a.links);
+  hipLaunchKernelGGL(rk.solve, dim3(unsigned(p.nregions)), dim3(unsigned(64 * rk.waves)), lds, stream, a);
+  AGD_HIP_TRY(hipGetLastError());
+  AGD_HIP_TRY(hipEventRecord(ws.ev1, stream));
+  touched = true;
+  AGD_HIP_TRY(hipMemcpyAsync(ws.host_counts, a.ctl, kRegionCtl * 4, hipMemcpyDeviceToHost, stream));
+  AGD_HIP_TRY(hipStreamSynchronize(stream));
+  const uint32_t* c = reinterpret_cast<const uint32_t*>(ws.host_counts);
+  if (c[kRegionFinished] != 1u) return AGD_OK;
+  taken = true;
+  if (stats) {
+    float ms = 0.f;
+    AGD_HIP_TRY(hipEventElapsedTime(&ms, ws.ev0, ws.ev1));
+    uint64_t visits = 0;
+    std::memcpy(&visits, c + kRegionVisits, sizeof visits);
+    stats->kernel_ms = d->time_launches ? ms : 0.;
+    stats->niter_o = c[kRegionRounds];
+    stats->tile_updates = int64_t(visits);
+    stats->cell_updates = int64_t(visits) * 64;
+    stats->launches = c[kRegionRounds];
+    stats->gpu_ms = ms;
+    stats->converged = 1;
+    stats->grid_blocks = p.nregions;
+  }
+  return AGD_OK;
+}
+
 template <class S>
 static int solve_impl(Workspace& ws, const agd_eikonal_desc* d, const agd_eikonal_io* io,
                       agd_eikonal_stats* stats, hipStream_t stream) {
@@ -639,6 +790,19 @@ static int solve_impl(Workspace& ws, const agd_eikonal_desc* d, const agd_eikona
     AGD_HIP_TRY(hipGetLastError());
   }
 
+  // The one-launch solve takes what the fast iterative method solves by default;
+  // a bound on the passes below the default one, passes timed or launched one
+  // by one, and the variants of the general kernel that it lacks stay here.
+  int32_t activate_all = d->activate_all;
+  if (!ws.fixed && d->solver == AGD_FIM && d->use_graph && !d->time_launches &&
+      (!pre || stored_scheme_model(d->model)) && !order2 && !factor && !big && d->nitermax_o >= 2000) {
+    bool taken = false, touched = false;
+    const int st = region_impl<S>(ws, a, d, io, stats, stream, taken, touched);
+    if (st) return st;
+    if (taken) return AGD_OK;
+    if (touched) activate_all = 1;
+  }
+
   auto init = [&](Workspace* ws) -> int {
     a.w.lists = ws->lists;
     a.w.counts = ws->counts;
@@ -658,7 +822,7 @@ static int solve_impl(Workspace& ws, const agd_eikonal_desc* d, const agd_eikona
     } else {
       const uint32_t* trig = io->trigger ? io->trigger : io->seeds;
       hipLaunchKernelGGL(ks.init, dim3(unsigned(ceil_div(g.ntiles, 64))), dim3(64), 0, stream, trig,
-                         g, d->activate_all, ws->stamp, ws->lists, ws->counts, a.w.shard_cap);
+                         g, activate_all, ws->stamp, ws->lists, ws->counts, a.w.shard_cap);
     }
     if (bab) {
       a.bab.ctl = ws->bab;

@@ -1,0 +1,848 @@
+// region_kernels.hpp -- the whole fixed-point iteration in one launch, for
+// grids whose values fit the LDS of the device.
+//
+// The pass solver (worklist.hpp) pays 7 to 13 us a pass on fronts of a few
+// hundred tiles: a kernel boundary, the list counters, the list entry, the
+// cell loads, the stencil, the gathers and two atomics follow one another.
+// Here every tile (8x8 or 4x4x4 cells, one lane per cell) belongs to one wave
+// of one workgroup for the whole solve, all workgroups resident at once, one
+// per compute unit.  A workgroup's tiles ("region") are boxes of one tile per
+// wave; their values stay in LDS, and no queue, lock or workgroup barrier is
+// needed:
+//   * a key per tile (LDS) says that it is to be visited, and how early: the
+//     least value that changed around it;
+//   * a visit loads the tile's stencil (built once by region_setup: weights
+//     and, per neighbour, an LDS slot or a grid index outside the region),
+//     relaxes the tile until it stops changing, stores it, and marks the tiles
+//     that read it (region_links: exactly those, diagonal ones included);
+//   * marks that leave the region increment a counter per tile in device
+//     memory, after the stores they announce have completed; a wave polls the
+//     counters of its tiles when it has nothing else to do.
+// Values only decrease and a tile has one writer, so a read of a neighbour's
+// older value is a supersolution that a later mark corrects: the fixed point
+// is that of the pass solver.  Values that cross regions are read and written
+// with device-scope accesses.
+//
+// Termination: a region that has nothing dirty or being visited, and whose own
+// marks have been delivered, publishes how many marks from outside it has
+// taken in.  Region 0's first wave, when idle, reads what all the regions
+// published, then all the counters.  Equal sums mean that every mark ever sent
+// was taken in by a region that has since been at rest; a region leaves its
+// rest only by taking in a mark that it has not published yet, so none is at
+// work and none will be.  That wave then writes every region's `done` word.
+//
+// Every wait is bounded: the workgroups first agree that all of them are
+// resident (a word decided once, go or abort, within start_ticks), and every
+// idle wave leaves after limit_ticks.  The caller then finishes with the pass
+// solver from the values reached.
+//
+// What bounds it: the chain of visits along the front (a wave is idle for 80 %
+// of the solve): a visit takes 3 to 5 us with its 300 (Isotropic2) to 5500
+// (Elastica2) cycles a sweep, a mark across regions 3 to 4 us more.  Measured,
+// pass solver -> here (solve alone, us): isotropic2 61 x 48 221 -> 60, 512^2
+// 1390 -> 450; riemann2 389 x 257 FP64 1580 -> 1070; isotropic3 121 x 77 x 95 with walls 1330 -> 640;
+// riemann3 97 x 101 x 89 1500 -> 1140; tti2 301 x 263 8430 -> 1510;
+// reedssheppforward2 96 x 80 x 64 1750 -> 960; elastica2 64 x 56 x 48 4930 ->
+// 1650.  One contiguous box per workgroup instead of many small ones left
+// most compute units idle: riemann3 took 1580.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include "common.hpp"
+#include "device.hpp"
+
+namespace agd {
+
+// Control words of a solve (device memory, zeroed before the launch).
+constexpr int kRegionArrived = 0;
+constexpr int kRegionGo = 32;        // 0 undecided, 1 go, 2 abort
+constexpr int kRegionFinished = 33;  // 1: the fixed point was reached
+constexpr int kRegionRounds = 34;    // largest number of visits of one wave
+constexpr int kRegionVisits = 64;    // uint64: tile visits
+constexpr int kRegionCtl = 96;
+constexpr int kRegionLine = 32;      // words between the regions' done words
+
+// How the grid is cut: into boxes of one tile per wave (RegionTraits), dealt
+// in turn to the regions, so that a front that crosses a part of the grid
+// still finds work on every compute unit.
+struct RegionPlan {
+  int32_t shape[3];   // cells
+  int32_t ntl[3];     // tiles
+  int32_t nbox[3];    // boxes
+  int32_t nboxes, nregions;
+  int32_t ntot;       // tiles of a region: its boxes times the waves
+  int32_t periodic;
+  int32_t ls[3];      // log2 of the storage tile shape
+  int32_t so[3];      // storage tiles
+  int32_t lsum;
+};
+
+template <class S> struct RegionArgs {
+  RegionPlan p;
+  S* u;
+  const S* geom;
+  const S* sw;            // stored schemes (TTI, curvature models)
+  const int32_t* scode;
+  const S* rhs;
+  const uint32_t* seeds;
+  const uint32_t* trigger;
+  const uint8_t* wall;
+  int64_t size_tot;
+  S iso_w[3];
+  S atol, rtol;
+  int32_t activate_all;
+  float window;            // tiles of key up to the region's least + window * (a tile's spread)
+  int32_t convex;
+  char* blocks;            // per tile: NCOMP rows of 64 entries
+  uint64_t* readers;       // per tile: window bits of the tiles that read it
+  int32_t* links;          // per tile: 64 targets, see region_links
+  uint32_t* ctl;           // kRegionCtl words
+  uint32_t* rest;          // per region: marks taken in at its last rest, plus 1; 0 before
+  uint32_t* done;          // per region, kRegionLine words apart
+  uint32_t* marks;         // per tile (see region_mark): marks from other regions
+  int64_t start_ticks, limit_ticks;
+};
+
+// Boxes (P tiles a side, one tile per wave), tiles, and the window of tile
+// offsets in which the readers of a tile are tracked: 3 tiles each way in 2D
+// (24 cells), 1 in 3D, and (2, 2, 1) without its edges for the curvature
+// models, whose offsets reach 5 cells in the plane.  One lane per offset, the
+// last lane left out.
+//   Box of 16 waves in 3D: 2 x 2 x 4 tiles (8 x 8 x 16 cells), but 4 x 4 x 1
+// for the curvature models: fewer of their long planar offsets leave the box
+// (ReedsSheppForward2 96 x 80 x 64: 1.23 -> 0.96 ms).
+template <int D, int W, bool CURV> struct RegionTraits {
+  static_assert(W == 8 || W == 16, "8 or 16 waves");
+  static constexpr bool FLAT = CURV && W == 16;
+  static constexpr int P0 = FLAT || (D == 2 && W == 16) ? 4 : 2;
+  static constexpr int P1 = FLAT || D == 2 ? 4 : 2;
+  static constexpr int P2 = FLAT || D == 2 ? 1 : (W == 16 ? 4 : 2);
+  static constexpr int LT = D == 2 ? 3 : 2;  // log2 of the tile side
+  static constexpr int NWIN = D == 2 ? 49 : (CURV ? 63 : 27);
+  static_assert(P0 * P1 * P2 == W, "one tile of the pattern per wave");
+  // Lane of a tile offset, -1 outside the window.
+  __device__ static inline int win_lane(const int* d) {
+    if constexpr (D == 2) {
+      return d[0] < -3 || d[0] > 3 || d[1] < -3 || d[1] > 3 ? -1 : (d[0] + 3) * 7 + d[1] + 3;
+    } else if constexpr (!CURV) {
+      return d[0] < -1 || d[0] > 1 || d[1] < -1 || d[1] > 1 || d[2] < -1 || d[2] > 1
+                 ? -1
+                 : ((d[0] + 1) * 3 + d[1] + 1) * 3 + d[2] + 1;
+    } else {
+      // 21 offsets a layer: the 5 x 5 square but for its corners
+      const int sq = (d[0] + 2) * 5 + d[1] + 2;
+      const bool out = d[0] < -2 || d[0] > 2 || d[1] < -2 || d[1] > 2 || d[2] < -1 || d[2] > 1 || sq == 0 ||
+                       sq == 4 || sq == 20 || sq == 24;
+      return out ? -1 : (d[2] + 1) * 21 + sq - 1 - (sq > 4 ? 1 : 0) - (sq > 20 ? 1 : 0);
+    }
+  }
+  // Offset of lane < NWIN.  The opposite offset is that of lane NWIN - 1 - lane.
+  __device__ static inline void win_offset(int lane, int* d) {
+    if constexpr (D == 2) {
+      d[0] = lane / 7 - 3;
+      d[1] = lane % 7 - 3;
+    } else if constexpr (!CURV) {
+      d[0] = lane / 9 - 1;
+      d[1] = lane / 3 % 3 - 1;
+      d[2] = lane % 3 - 1;
+    } else {
+      const int q = lane % 21;
+      const int sq = q + 1 + (q > 2 ? 1 : 0) + (q > 17 ? 1 : 0);
+      d[0] = sq / 5 - 2;
+      d[1] = sq % 5 - 2;
+      d[2] = lane / 21 - 1;
+    }
+  }
+};
+
+// Entries of a tile's block, per cell: weights, neighbour codes, [shifts],
+// rhs (scalar type), then own storage index and, with several sub-schemes,
+// the min/max flag.
+template <class S, int MODEL, int D> struct RegionScheme {
+  using MT = ModelTraits<MODEL, D>;
+  static constexpr int NS = MT::NSYM;
+  static constexpr int NSIDE = 2 * (NS - MT::NFWD);      // codes of the symmetric offsets
+  static constexpr int NC = MT::NMIX * (NSIDE + MT::NFWD);
+  static constexpr int NW = MODEL == AGD_ISOTROPIC ? 0 : MT::NMIX * NS;
+  static constexpr int NSH = MT::DRIFT ? NS : 0;
+  static constexpr int NI32 = NC + 1 + (MT::NMIX > 1 ? 1 : 0);
+  static constexpr int NREAL = NW + NSH + 1;
+  static constexpr int BYTES = 64 * (NREAL * int(sizeof(S)) + NI32 * 4);  // of a tile
+  // 16 waves (4 per SIMD) where the visit fits 128 registers, else 8
+  static constexpr int W = (MODEL == AGD_TTI || MODEL == AGD_ELASTICA2) ? 8 : 16;
+  using RT = RegionTraits<D, W, MT::CURV>;
+  // Relaxations of a visit at most.  Cheap ones run on (a visit costs about 3000
+  // cycles beside them); dear ones wait for better inputs.  Measured with 2,
+  // 4, 8, 12: isotropic2 512^2 1830, 917, 516, 468 us; riemann3 97 x 101 x 89 1220,
+  // 1136, -, 1393 us; elastica2 64 x 56 x 48 1654, 1857, 2900, 3600 us; riemann2
+  // 389 x 257 in FP64 1071, 1269, 1894, 2766 us.
+  static constexpr int SWEEPS = sizeof(S) == 8 || NS * MT::NMIX >= 30 ? 2 : (NS * MT::NMIX >= 6 ? 4 : 12);
+  // the stencil of the last tile visited stays in registers
+  static constexpr bool KEEP = NC <= 8 && sizeof(S) == 4;
+  // LDS of a region of ntot tiles: their values, +inf, and per wave the
+  // values of a tile's neighbours outside the region
+  static constexpr size_t lds(int ntot) { return (size_t(ntot) * 64 + 64 + size_t(W) * NC * 64) * sizeof(S); }
+};
+
+constexpr int32_t kRegionNone = INT32_MIN;  // code: no neighbour
+
+// Order-preserving image of a value; kKeyNone is above all of them.
+constexpr uint32_t kKeyNone = 0xffffffffu;
+__device__ inline uint32_t key_of(float v) {
+  const uint32_t i = __float_as_uint(v);
+  return (i & 0x80000000u) ? ~i : (i | 0x80000000u);
+}
+__device__ inline float key_value(uint32_t k) {
+  return __uint_as_float((k & 0x80000000u) ? (k & 0x7fffffffu) : ~k);
+}
+// Smallest of the wave's values, in every lane.
+__device__ inline uint32_t wave_min(uint32_t v) {
+  const int none = int(kKeyNone);
+  v = min(v, uint32_t(__builtin_amdgcn_update_dpp(none, int(v), 0x111, 0xf, 0xf, false)));
+  v = min(v, uint32_t(__builtin_amdgcn_update_dpp(none, int(v), 0x112, 0xf, 0xf, false)));
+  v = min(v, uint32_t(__builtin_amdgcn_update_dpp(none, int(v), 0x114, 0xf, 0xf, false)));
+  v = min(v, uint32_t(__builtin_amdgcn_update_dpp(none, int(v), 0x118, 0xf, 0xf, false)));
+  v = min(v, uint32_t(__builtin_amdgcn_update_dpp(none, int(v), 0x142, 0xa, 0xf, false)));
+  v = min(v, uint32_t(__builtin_amdgcn_update_dpp(none, int(v), 0x143, 0xc, 0xf, false)));
+  return uint32_t(__builtin_amdgcn_readlane(int(v), 63));
+}
+
+// Index of a tile's counter: the tiles of a wave follow each other.
+template <int W> __device__ inline int region_mark(const RegionPlan& p, int r, int l) {
+  return r * p.ntot + (l % W) * (p.ntot / W) + l / W;
+}
+
+template <class T> __device__ inline T ld_agent(const T* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <class T> __device__ inline void st_agent(T* p, T v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Every earlier access of the wave to device memory has completed.
+__device__ inline void wait_memory() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+__device__ inline void compiler_fence() { asm volatile("" ::: "memory"); }
+
+template <int D> __device__ __host__ inline int region_storage(const RegionPlan& p, const int* x) {
+  int to = x[0] >> p.ls[0];
+  int in = x[0] & ((1 << p.ls[0]) - 1);
+#pragma unroll
+  for (int c = 1; c < D; ++c) {
+    to = to * p.so[c] + (x[c] >> p.ls[c]);
+    in = (in << p.ls[c]) | (x[c] & ((1 << p.ls[c]) - 1));
+  }
+  return (to << p.lsum) | in;
+}
+
+// Cell of a storage index.
+template <int D> __device__ __host__ inline void region_cell(const RegionPlan& p, int n, int* x) {
+  int to = n >> p.lsum, in = n & ((1 << p.lsum) - 1);
+#pragma unroll
+  for (int c = D - 1; c >= 0; --c) {
+    const int q = c > 0 ? to / p.so[c] : 0;
+    x[c] = ((to - q * p.so[c]) << p.ls[c]) | (in & ((1 << p.ls[c]) - 1));
+    to = q;
+    in >>= p.ls[c];
+  }
+}
+
+// Region and place in it (l = box of the region * W + wave) of a tile.
+template <int D, class RT>
+__device__ __host__ inline int region_of(const RegionPlan& p, const int* t, int& l) {
+  constexpr int P[3] = {RT::P0, RT::P1, RT::P2};
+  constexpr int W = RT::P0 * RT::P1 * RT::P2;
+  int box = 0, w = 0;
+#pragma unroll
+  for (int c = 0; c < D; ++c) {
+    box = box * p.nbox[c] + int(unsigned(t[c]) / unsigned(P[c]));
+    w = w * P[c] + (t[c] & (P[c] - 1));
+  }
+  const int b = box / p.nregions;
+  l = b * W + w;
+  return box - b * p.nregions;
+}
+
+// Tile of place l of region r; false outside the grid.
+template <int D, class RT>
+__device__ __host__ inline bool region_tile(const RegionPlan& p, int r, int l, int* t) {
+  constexpr int P[3] = {RT::P0, RT::P1, RT::P2};
+  constexpr int W = RT::P0 * RT::P1 * RT::P2;
+  int w = l % W, box = (l / W) * p.nregions + r;
+  bool in = box < p.nboxes;
+#pragma unroll
+  for (int c = D - 1; c >= 0; --c) {
+    const int q = c > 0 ? box / p.nbox[c] : 0;
+    t[c] = (box - q * p.nbox[c]) * P[c] + (w & (P[c] - 1));
+    in = in && t[c] < p.ntl[c];
+    w /= P[c];
+    box = q;
+  }
+  return in;
+}
+
+// ------------------------------------------------------------------ setup
+// One wave per tile: the tile's block, its readers' window bits, the seeds'
+// values and the initial dirty bits.
+template <class S, int MODEL, int D>
+__global__ void __launch_bounds__(256) region_setup(RegionArgs<S> a) {
+  using MT = ModelTraits<MODEL, D>;
+  using RS = RegionScheme<S, MODEL, D>;
+  constexpr int W = RS::W;
+  using RT = typename RS::RT;
+  constexpr int NS = MT::NSYM;
+  const RegionPlan& p = a.p;
+  const int lane = threadIdx.x & 63;
+  const int sub = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
+  if (sub >= p.nregions * p.ntot) return;
+  const int r = sub / p.ntot, l = sub - r * p.ntot;
+  int t[3] = {0, 0, 0};
+  if (!region_tile<D, RT>(p, r, l, t)) return;  // beyond the grid: never marked
+  int x[3] = {0, 0, 0};
+  if constexpr (D == 2) {
+    x[0] = t[0] * 8 + (lane >> 3);
+    x[1] = t[1] * 8 + (lane & 7);
+  } else {
+    x[0] = t[0] * 4 + (lane >> 4);
+    x[1] = t[1] * 4 + ((lane >> 2) & 3);
+    x[2] = t[2] * 4 + (lane & 3);
+  }
+  bool dom = true;
+#pragma unroll
+  for (int c = 0; c < D; ++c) dom = dom && x[c] < p.shape[c];
+  const int n = dom ? region_storage<D>(p, x) : 0;
+  const S rhs = dom ? a.rhs[n] : inf_v<S>();
+  const bool seed = dom && ((a.seeds[n >> 5] >> (n & 31)) & 1u);
+  if (seed) a.u[n] = rhs;
+  const bool live = dom && !seed;
+  const bool trig = dom && (a.activate_all || ((a.trigger[n >> 5] >> (n & 31)) & 1u));
+
+  S* real = reinterpret_cast<S*>(a.blocks + int64_t(sub) * RS::BYTES) + lane;
+  int32_t* ints = reinterpret_cast<int32_t*>(a.blocks + int64_t(sub) * RS::BYTES + 64 * RS::NREAL * sizeof(S)) + lane;
+
+  // The code of neighbour cell y (already wrapped, in the domain), and the
+  // window bit of its tile.
+  uint64_t reads = 0;
+  auto encode = [&](const int* y) -> int32_t {
+    int ty[3] = {0, 0, 0};
+    int lane_y = 0;
+#pragma unroll
+    for (int c = 0; c < D; ++c) {
+      ty[c] = y[c] >> RT::LT;
+      lane_y = (lane_y << RT::LT) | (y[c] & ((1 << RT::LT) - 1));
+    }
+    // (most neighbours lie in the own box)
+    constexpr int P[3] = {RT::P0, RT::P1, RT::P2};
+    bool home = true;
+    int lw = 0;
+#pragma unroll
+    for (int c = 0; c < D; ++c) {
+      home = home && ((ty[c] ^ t[c]) & ~(P[c] - 1)) == 0;
+      lw = lw * P[c] + (ty[c] & (P[c] - 1));
+    }
+    int ly = (l / W) * W + lw;
+    if (!home) home = region_of<D, RT>(p, ty, ly) == r;
+    int d[3] = {0, 0, 0};
+    bool self = true;
+#pragma unroll
+    for (int c = 0; c < D; ++c) {
+      d[c] = ty[c] - t[c];
+      if ((p.periodic >> c) & 1) {  // the nearer way round
+        if (2 * d[c] > p.ntl[c]) d[c] -= p.ntl[c];
+        if (2 * d[c] < -p.ntl[c]) d[c] += p.ntl[c];
+      }
+      self = self && d[c] == 0;
+    }
+    const int win = RT::win_lane(d);
+    if (win >= 0 && !self) reads |= uint64_t(1) << win;
+    return home ? -1 - (ly * 64 + lane_y) : region_storage<D>(p, y);
+  };
+
+  if constexpr (MT::STORED) {
+    const int64_t N = a.size_tot;
+    const bool mix_min = dom && a.scode[int64_t(MT::NMIX * 2 * NS) * N + n] != 0;
+#pragma unroll 1
+    for (int m = 0; m < MT::NMIX; ++m) {
+      int q = m * (RS::NSIDE + MT::NFWD);
+#pragma unroll 1
+      for (int k = 0; k < NS; ++k) {
+        const S w = live ? a.sw[int64_t(m * NS + k) * N + n] : S(0);
+        real[64 * (m * NS + k)] = w;
+        // curvature models: an offset of weight 0 takes no part in the update
+        const bool off = !live || (MT::CURV && !(w > S(0)));
+#pragma unroll 1
+        for (int sd = (k >= NS - MT::NFWD ? 1 : 0); sd < 2; ++sd, ++q) {
+          const int c = off ? -1 : a.scode[int64_t(m * 2 * NS + 2 * k + sd) * N + n];
+          int32_t code = kRegionNone;
+          if (c != -1) {
+            int y[3] = {0, 0, 0};
+            region_cell<D>(p, c >= 0 ? c : ((n >> p.lsum) << p.lsum) + (-2 - c), y);
+            code = encode(y);
+          }
+          ints[64 * q] = code;
+        }
+      }
+    }
+    if constexpr (MT::NMIX > 1) ints[64 * (RS::NC + 1)] = mix_min ? 1 : 0;
+  } else {
+    constexpr int NG = MT::NGEOM;
+    S geo[NG > 0 ? NG : 1];
+#pragma unroll
+    for (int k = 0; k < NG; ++k) geo[k] = dom ? a.geom[int64_t(k) * a.size_tot + n] : inf_v<S>();
+    Stencil<S, MODEL, D> st;
+    make_stencil<S, MODEL, D>(geo, a.iso_w, st);
+    const int wx = (a.wall && live) ? int(a.wall[n]) : 255;
+    auto wrapped = [&](int* y) -> bool {
+      bool ok = true;
+#pragma unroll
+      for (int c = 0; c < D; ++c) {
+        if ((p.periodic >> c) & 1) y[c] = mod_pos(y[c], p.shape[c]);
+        else ok = ok && y[c] >= 0 && y[c] < p.shape[c];
+      }
+      return ok;
+    };
+#pragma unroll 1
+    for (int j = 0; j < RS::NC; ++j) {
+      // (selection by comparison keeps the stencil in registers)
+      int e[3] = {0, 0, 0};
+#pragma unroll
+      for (int k = 0; k < NS; ++k)
+        if (k == j >> 1)
+#pragma unroll
+          for (int c = 0; c < D; ++c) e[c] = (j & 1) ? st.e[k][c] : -st.e[k][c];
+      int32_t code = kRegionNone;
+      if (live) {
+        bool vis = true;
+        if (a.wall && wx != 255) {
+          vis = visible<D>(e, wx, [&](const int* w) -> int {
+            int y[3] = {x[0] + w[0], x[1] + w[1], x[2] + w[2]};
+            return wrapped(y) ? int(a.wall[region_storage<D>(p, y)]) : 255;
+          });
+        }
+        int y[3] = {x[0] + e[0], x[1] + e[1], x[2] + e[2]};
+        if (vis && wrapped(y)) code = encode(y);
+      }
+      ints[64 * j] = code;
+    }
+#pragma unroll
+    for (int k = 0; k < RS::NW; ++k) real[64 * k] = st.w[k];
+#pragma unroll
+    for (int k = 0; k < RS::NSH; ++k) real[64 * (RS::NW + k)] = st.shift[k];
+  }
+  real[64 * (RS::NREAL - 1)] = rhs;
+  ints[64 * RS::NC] = dom ? n : -1;
+
+  // readers: this tile reads the tiles of `reads`
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) reads |= __shfl_xor(reads, o);
+  if (lane < RT::NWIN && ((reads >> lane) & 1)) {
+    int d[3] = {0, 0, 0}, ty[3] = {0, 0, 0};
+    RT::win_offset(lane, d);
+#pragma unroll
+    for (int c = 0; c < D; ++c) {
+      ty[c] = t[c] + d[c];
+      if ((p.periodic >> c) & 1) ty[c] = mod_pos(ty[c], p.ntl[c]);
+    }
+    int ly;
+    const int ry = region_of<D, RT>(p, ty, ly);
+    atomicOr(reinterpret_cast<unsigned long long*>(a.readers + int64_t(ry) * p.ntot + ly),
+             1ull << (RT::NWIN - 1 - lane));
+  }
+  // (the first mark of a tile comes from outside too)
+  if (__any(trig) && lane == 0) a.marks[region_mark<W>(p, r, l)] = 1;
+}
+
+// The targets of a tile's marks, one per window offset: place l of the own
+// region, (region + 1) << 10 | l of another, -1 none.
+template <int D, class RT>
+__global__ void __launch_bounds__(256) region_links(RegionPlan p, const uint64_t* readers, int32_t* links) {
+  const int lane = threadIdx.x & 63;
+  const int sub = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
+  if (sub >= p.nregions * p.ntot) return;
+  const int r = sub / p.ntot, l = sub - r * p.ntot;
+  int t[3] = {0, 0, 0};
+  if (!region_tile<D, RT>(p, r, l, t)) return;
+  int32_t link = -1;
+  if (lane < RT::NWIN && ((readers[sub] >> lane) & 1)) {
+    int d[3] = {0, 0, 0}, ty[3] = {0, 0, 0};
+    RT::win_offset(lane, d);
+#pragma unroll
+    for (int c = 0; c < D; ++c) {
+      ty[c] = t[c] + d[c];
+      if ((p.periodic >> c) & 1) ty[c] = mod_pos(ty[c], p.ntl[c]);
+    }
+    int ly;
+    const int ry = region_of<D, RT>(p, ty, ly);
+    link = ry == r ? ly : ((ry + 1) << 10 | ly);
+  }
+  links[int64_t(sub) * 64 + lane] = link;
+}
+
+// ------------------------------------------------------------------ update
+// min and max of two values neither of which is a NaN unless noted: one
+// instruction each (fminf would first quiet its operands).  A NaN first or
+// second operand gives the other one.
+__device__ inline float min2(float a, float b) {
+  float r;
+  asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+__device__ inline float max2(float a, float b) {
+  float r;
+  asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+__device__ inline double min2(double a, double b) { return b < a ? b : a; }
+
+// Pairs in increasing order of v (the networks of sort_pairs; the order of
+// equal values is free).
+struct CexMin {
+  template <class S> __device__ static inline void swap(S& vi, S& wi, S& vj, S& wj) {
+    if constexpr (sizeof(S) == 4) {
+      const bool keep = vi < vj;
+      const S c = keep ? wi : wj;
+      wj = keep ? wj : wi;
+      wi = c;
+      const S lo = min2(vi, vj);
+      vj = max2(vi, vj);
+      vi = lo;
+    } else {
+      cex(vi, wi, vj, wj);
+    }
+  }
+};
+
+// hfm_solve for a value that only decreases: min(u, solution of
+// sum_k w_k (u - v_k)_+^2 = rhs^2), given nrhs2 = -rhs^2.  Where there is no
+// solution (no finite v, or no weight) the quadratic ends in a NaN or +inf,
+// which the minimum passes over.  A value at which the quadratic of the
+// smaller ones is positive leaves the active set by itself: at the larger
+// values after it the quadratic is larger still.
+template <class S, int N> __device__ inline S hfm_lower(S (&v)[N], S (&w)[N], S nrhs2, S u) {
+  sort_pairs_by<CexMin, S, N>(v, w);
+  const S vmin = v[0];
+  S a = w[0], b = S(0), c = nrhs2;
+#pragma unroll
+  for (int k = 1; k < N; ++k) {
+    const S t = v[k] - vmin;
+    const bool out = fma_(fma_(a, t, S(-2) * b), t, c) > S(0);
+    const S wk = out ? S(0) : w[k];
+    const S tk = out ? S(0) : t;
+    const S wt = wk * tk;
+    a += wk;
+    b += wt;
+    c = fma_(wt, tk, c);
+  }
+  const S delta = fma_(b, b, -(a * c));
+  const S root = vmin + div_fast(b + sqrt_fast(delta > S(0) ? delta : S(0)), a);
+  return min2(u, root);
+}
+
+// ------------------------------------------------------------------ solve
+template <class S, int MODEL, int D>
+__global__ void __launch_bounds__((64 * RegionScheme<S, MODEL, D>::W))
+    region_solve(RegionArgs<S> a) {
+  using MT = ModelTraits<MODEL, D>;
+  using RS = RegionScheme<S, MODEL, D>;
+  constexpr int W = RS::W;
+  using RT = typename RS::RT;
+  constexpr int NS = MT::NSYM;
+  const RegionPlan& p = a.p;
+  extern __shared__ __align__(16) char region_lds[];
+  S* const us = reinterpret_cast<S*>(region_lds);  // ntot * 64 values, then +inf
+  __shared__ uint32_t key[W * 32];  // per tile (w * 32 + b): least change it has to see, or kKeyNone
+  __shared__ uint32_t wkey[W];      // per wave: least key of its tiles, the visited one included
+  // low half: marked tiles and visits not accounted for; high half: marks
+  // from outside taken in
+  __shared__ unsigned long long account;
+  __shared__ uint32_t go;
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = blockIdx.x;
+  const int none = p.ntot * 64;  // LDS slot of +inf
+  const int nbits = p.ntot / W;
+  const int64_t t0 = wall_clock64();
+
+  // ---- all workgroups resident?
+  if (threadIdx.x == 0) {
+    uint32_t* const g = a.ctl + kRegionGo;
+    const uint32_t at = __hip_atomic_fetch_add(a.ctl + kRegionArrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (at + 1 == uint32_t(p.nregions)) atomicCAS(g, 0u, 1u);
+    uint32_t v;
+    while ((v = ld_agent(g)) == 0) {
+      if (wall_clock64() - t0 > a.start_ticks) {
+        atomicCAS(g, 0u, 2u);
+        v = ld_agent(g);
+        break;
+      }
+      __builtin_amdgcn_s_sleep(2);
+    }
+    go = v;
+    account = W;
+  }
+  if (threadIdx.x < 64) us[none + lane] = inf_v<S>();
+  // own tiles' values
+  for (int b = 0; b < nbits; ++b) {
+    const int l = b * W + w;
+    int t[3];
+    S v = inf_v<S>();
+    if (region_tile<D, RT>(p, r, l, t)) {
+      const char* blk = a.blocks + (int64_t(r) * p.ntot + l) * RS::BYTES;
+      const int n = reinterpret_cast<const int32_t*>(blk + 64 * RS::NREAL * sizeof(S))[64 * RS::NC + lane];
+      if (n >= 0) v = a.u[n];
+    }
+    us[l * 64 + lane] = v;
+  }
+  if (lane < 32) key[w * 32 + lane] = kKeyNone;
+  if (lane == 0) wkey[w] = kKeyNone;
+  __syncthreads();
+  if (go != 1u) return;
+
+  // what a lane polls: the counter of the wave's tile b = lane; lane 63: done
+  const uint32_t* const poll = lane < nbits ? a.marks + region_mark<W>(p, r, lane * W + w)
+                                            : a.done + r * kRegionLine;
+  uint32_t seen = 0;  // marks taken in of tile b = lane
+  int owed = 1;       // visits not accounted for
+  int visits = 0;
+  int loaded = -1;      // the tile whose stencil the registers hold
+  uint32_t again = 0;   // tiles whose outside values are to be gathered again
+  uint32_t unsent = 0;  // tiles changed since they last marked other regions
+  float spread = inf_v<float>();  // of a tile's values, running mean
+  S wt[RS::NW > 0 ? RS::NW : 1], sh[RS::NSH > 0 ? RS::NSH : 1], nrhs2 = S(0);
+  int code[RS::NC], slot[RS::NC];
+  int own = -1, mix_min = 1, link = -1;
+  bool outside = false, remote = false;
+  const int ext = none + 64 + w * (RS::NC * 64) + lane;  // slot of outside neighbour j: ext + 64 j
+
+  for (;;) {
+    // ---- the tile of the least key, if no wave of the region works far below it
+    const uint32_t seen_key =
+        *const_cast<volatile uint32_t*>(lane < 32 ? &key[w * 32 + lane] : &wkey[lane & (W - 1)]);
+    compiler_fence();
+    uint32_t least, floor_key = kKeyNone;
+    if (nbits == 1) {
+      least = __builtin_amdgcn_readfirstlane(seen_key);
+    } else {
+      least = wave_min(lane < 32 ? seen_key : kKeyNone);
+      floor_key = wave_min(lane < 32 || (lane & (W - 1)) == w ? kKeyNone : seen_key);
+      if (lane == 0) wkey[w] = least == 0 ? kKeyNone : least;  // (0: a mark from outside, of no known value)
+    }
+    if (least == kKeyNone || key_value(least) > key_value(floor_key) + a.window * spread) {
+      // ---- idle: account for what was done, then wait for marks
+      if (owed && least == kKeyNone) {
+        wait_memory();
+        if (lane == 0) {
+          const unsigned long long old = atomicAdd(&account, (unsigned long long)(-(long long)owed));
+          if (uint32_t(old) == uint32_t(owed))
+            __hip_atomic_fetch_max(a.rest + r, uint32_t(old >> 32) + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        owed = 0;
+      }
+      const uint32_t now = ld_agent(poll);
+      bool local = false;
+      for (int i = 0; i < 4 && !local; ++i) {
+        __builtin_amdgcn_s_sleep(1);
+        const uint32_t k2 =
+            *const_cast<volatile uint32_t*>(lane < 32 ? &key[w * 32 + lane] : &wkey[lane & (W - 1)]);
+        local = __any(lane < 32 ? k2 != seen_key : (least != kKeyNone && k2 != seen_key));
+      }
+      if (local) continue;
+      const uint32_t got = uint32_t(__ballot(lane < nbits && now != seen));
+      if (got) {
+        uint32_t more = lane < nbits ? now - seen : 0u;
+        if (lane < nbits) seen = now;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) more += __shfl_xor(more, o);
+        if (lane == 0) atomicAdd(&account, ((unsigned long long)more << 32) + (unsigned long long)__popc(got));
+        if (lane < 32 && ((got >> lane) & 1) && atomicMin(&key[w * 32 + lane], 0u) != kKeyNone)
+          atomicAdd(&account, ~0ull);
+        again |= got;
+        continue;
+      }
+      if (__builtin_amdgcn_readlane(now, 63) != 0 || wall_clock64() - t0 > a.limit_ticks) break;
+      if (r == 0 && w == 0 && least == kKeyNone) {
+        // ---- the fixed point?
+        bool quiet = true;
+        uint32_t sum = 0;
+        for (int i = lane; i < p.nregions; i += 64) {
+          const uint32_t s = ld_agent(a.rest + i);
+          quiet = quiet && s != 0;
+          sum += s - 1;
+        }
+        wait_memory();
+        if (!__any(!quiet)) {
+          for (int i = lane; i < p.nregions * p.ntot; i += 64) sum -= ld_agent(a.marks + i);
+#pragma unroll
+          for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
+          if (sum == 0) {
+            for (int i = lane; i < p.nregions; i += 64) st_agent(a.done + i * kRegionLine, 1u);
+            if (lane == 0) st_agent(a.ctl + kRegionFinished, 1u);
+          }
+        }
+      }
+      continue;
+    }
+
+    // ---- visit it
+    // (a mark made between the read of its key and this write is taken in too:
+    // the values are read after it)
+    const int b = nbits == 1 ? 0 : __builtin_ctzll(__ballot(lane < 32 && seen_key == least));
+    if (lane == 0) key[w * 32 + b] = kKeyNone;
+    compiler_fence();
+    ++owed;
+    const int l = b * W + w;
+    if ((++visits & 63) == 0 && wall_clock64() - t0 > a.limit_ticks) break;
+    const bool load = !RS::KEEP || l != loaded;
+    const bool gather = load || ((again >> b) & 1);
+    again &= ~(1u << b);
+    if (load) {
+      loaded = l;
+      const char* blk = a.blocks + (int64_t(r) * p.ntot + l) * RS::BYTES;
+      const S* real = reinterpret_cast<const S*>(blk) + lane;
+      const int32_t* ints = reinterpret_cast<const int32_t*>(blk + 64 * RS::NREAL * sizeof(S)) + lane;
+#pragma unroll
+      for (int j = 0; j < RS::NC; ++j) code[j] = ints[64 * j];
+#pragma unroll
+      for (int k = 0; k < RS::NW; ++k) wt[k] = real[64 * k];
+#pragma unroll
+      for (int k = 0; k < RS::NSH; ++k) sh[k] = real[64 * (RS::NW + k)];
+      const S rhs = real[64 * (RS::NREAL - 1)];
+      nrhs2 = -rhs * rhs;
+      own = ints[64 * RS::NC];
+      if constexpr (MT::NMIX > 1) mix_min = ints[64 * (RS::NC + 1)];
+      link = a.links[(int64_t(r) * p.ntot + l) * 64 + lane];
+      remote = __any(link >= 1024);
+      bool out = false;
+#pragma unroll
+      for (int j = 0; j < RS::NC; ++j) {
+        out = out || code[j] >= 0;
+        slot[j] = code[j] >= 0 ? ext + 64 * j : (code[j] != kRegionNone ? -1 - code[j] : none);
+      }
+      outside = __any(out);
+    }
+    if (gather && outside) {
+      S g[RS::NC];
+#pragma unroll
+      for (int j = 0; j < RS::NC; ++j)
+        if (code[j] >= 0) g[j] = ld_agent(a.u + code[j]);
+#pragma unroll
+      for (int j = 0; j < RS::NC; ++j)
+        if (code[j] >= 0) us[ext + 64 * j] = g[j];
+    }
+    const int mine = l * 64 + lane;
+    const S u0 = us[mine];
+    S un = u0;
+    bool more = true;
+    // (two sweeps between two looks at whether anything changes; a cell that
+    // does not change writes its own value again)
+    for (int it = 0; it < RS::SWEEPS && more; it += 2) {
+      const S ub = un;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        compiler_fence();
+        S x[RS::NC];
+#pragma unroll
+        for (int j = 0; j < RS::NC; ++j) x[j] = us[slot[j]];
+        if constexpr (RS::NC <= 12) {
+          // (keeps every read ahead of its first use)
+#pragma unroll
+          for (int j = 0; j < RS::NC; ++j) asm volatile("" ::"v"(x[j]));
+        }
+        S best = mix_min ? inf_v<S>() : -inf_v<S>();
+#pragma unroll
+        for (int m = 0; m < MT::NMIX; ++m) {
+          S v[NS], ww[NS];
+#pragma unroll
+          for (int k = 0; k < NS; ++k) {
+            const int q = m * (RS::NSIDE + MT::NFWD) + (k < NS - MT::NFWD ? 2 * k : RS::NSIDE + k - (NS - MT::NFWD));
+            v[k] = x[q];
+            if (k < NS - MT::NFWD) {
+              if constexpr (MT::DRIFT) v[k] = min2(x[q] + sh[k], x[q + 1] - sh[k]);
+              else v[k] = min2(x[q], x[q + 1]);
+            }
+            ww[k] = MODEL == AGD_ISOTROPIC ? a.iso_w[k < 3 ? k : 0] : wt[m * NS + k];
+          }
+          if constexpr (MT::NMIX > 1) {
+            // (no solution counts as +inf, also in a maximum)
+            const S um = hfm_lower<S, NS>(v, ww, nrhs2, inf_v<S>());
+            if ((mix_min != 0) == (best > um)) best = um;
+          } else {
+            un = hfm_lower<S, NS>(v, ww, nrhs2, un);
+          }
+        }
+        if constexpr (MT::NMIX > 1) un = min2(un, best);
+        us[mine] = un;
+      }
+      more = __any(un < ub);
+    }
+    compiler_fence();
+    if (own >= 0 && un < u0) st_agent(a.u + own, un);
+    const S diff = abs_(u0 - un);
+    const S tol = a.atol + a.rtol * abs_(un);
+    const bool changed = !(isnan_(diff) || diff <= tol);
+    const bool rest = !(more && __any(changed));
+    if (__any(changed)) {
+      // ---- marks: the tiles of the region that read this one, and itself if
+      // it was cut short
+      const uint32_t kc = nbits == 1 ? 1u : wave_min(changed ? key_of(float(un)) : kKeyNone);
+      const bool here = (link >= 0 && link < 1024) || (!rest && lane == 63);
+      const int tl = (lane == 63) ? l : link;
+      if (here) {
+        atomicAdd(&account, 1ull);
+        if (atomicMin(&key[(tl % W) * 32 + tl / W], kc) != kKeyNone) atomicAdd(&account, ~0ull);
+      }
+      if (remote) unsent |= 1u << b;
+      if (rest && nbits > 1 && (visits & 3) == 0) {
+        const float hi = key_value(~wave_min(~key_of(own >= 0 ? float(un) : -inf_v<float>())));
+        const float lo = key_value(wave_min(own >= 0 ? key_of(float(un)) : kKeyNone));
+        const float sp = hi - lo;
+        if (sp < inf_v<float>()) spread = spread == inf_v<float>() ? sp : 0.875f * spread + 0.125f * sp;
+      }
+    }
+    if (rest && ((unsent >> b) & 1)) {
+      // ---- a tile at rest marks the readers in other regions
+      unsent &= ~(1u << b);
+      wait_memory();
+      if (link >= 1024)
+        __hip_atomic_fetch_add(a.marks + region_mark<W>(p, (link >> 10) - 1, link & 1023), 1u, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
+  if (lane == 0) {
+    atomicAdd(reinterpret_cast<unsigned long long*>(a.ctl + kRegionVisits), (unsigned long long)visits);
+    atomicMax(a.ctl + kRegionRounds, uint32_t(visits));
+  }
+}
+
+// ------------------------------------------------------------------ tables
+// Kernels of one (model, dimension); null where there are none.
+template <class S> struct RegionKernels {
+  void (*setup)(RegionArgs<S>) = nullptr;
+  void (*links)(RegionPlan, const uint64_t*, int32_t*) = nullptr;
+  void (*solve)(RegionArgs<S>) = nullptr;
+  int waves = 0;       // of a workgroup of solve
+  int box[3] = {1, 1, 1};  // tiles of a box
+  int tile_bytes = 0;  // of a tile's block
+  size_t (*lds)(int) = nullptr;  // of a workgroup, for so many tiles
+};
+
+template <class S, int MODEL, int D> RegionKernels<S> make_region_kernels() {
+  using RS = RegionScheme<S, MODEL, D>;
+  RegionKernels<S> k;
+  k.setup = region_setup<S, MODEL, D>;
+  k.links = region_links<D, typename RS::RT>;
+  k.solve = region_solve<S, MODEL, D>;
+  k.waves = RS::W;
+  k.box[0] = RS::RT::P0;
+  k.box[1] = RS::RT::P1;
+  k.box[2] = RS::RT::P2;
+  k.tile_bytes = RS::BYTES;
+  k.lds = RS::lds;
+  return k;
+}
+
+// Defined (and instantiated) in region_<group>.hip.
+template <class S> RegionKernels<S> region_plain(int model, int d);   // Isotropic, Diagonal
+template <class S> RegionKernels<S> region_metric(int model, int d);  // Riemann, Rander
+RegionKernels<float> region_stored(int model, int d);                 // TTI2, curvature models
+
+}  // namespace agd

@@ -62,6 +62,8 @@ struct Workspace {
   int32_t* tile_inst = nullptr;    // batched solves: tile -> instance (tinst_cap)
   void* ftab = nullptr;            // TTI source factorization: shift table (ftab_bytes)
   size_t ftab_bytes = 0;
+  void* region = nullptr;          // one-launch solve: control words, tile blocks (region_bytes)
+  size_t region_bytes = 0;
   int64_t tile_cap = 0, shard_cap = 0, hist_cap = 0, inst_cap = 0, tinst_cap = 0;
   // Host side.  host_counts: pinned (owned) or host_local (fixed region),
   // 2 * kRow entries, two chunks in flight.
@@ -94,6 +96,8 @@ struct Workspace {
   int ensure_batch(int64_t ninst, int64_t ntiles, size_t inst_bytes);
   // TTI source factorization: a shift table of at least `bytes`.
   int ensure_ftab(size_t bytes);
+  // One-launch solve: a buffer of at least `bytes`.
+  int ensure_region(size_t bytes);
   // Frees everything owned (no-op for a fixed region).
   void release();
   // Lays the buffers out in [base, base + bytes) (fixed region); AGD_EINVAL

@@ -149,6 +149,10 @@ typedef struct agd_eikonal_io {
   int64_t scheme_codes_len;
 } agd_eikonal_io;
 
+/* A FIM solve of a grid that fits the LDS of the device runs as one launch
+ * (csrc/region_kernels.hpp), unless nitermax_o is below 2000, use_graph is 0,
+ * time_launches is set, or another such solve is running on the device; it
+ * reports as niter_o and launches the visits of its busiest wave. */
 typedef struct agd_eikonal_stats {
   int64_t niter_o;        /* grid-level passes with a non-empty tile list */
   int64_t tile_updates;   /* tile visits summed over passes               */
