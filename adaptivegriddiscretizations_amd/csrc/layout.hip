@@ -28,9 +28,19 @@ struct LayoutDesc {
   int32_t shape_i[3];
   int32_t shape_o[3];
   int32_t size_i;
+  int32_t ls[3], lsize;  // log2 of the tile shape and size (powers of two)
+  int32_t form;          // of tiled_to_cell
   int64_t size_tot;
   int64_t ncell;
 };
+
+// How an index is split into its tile and its place in it.  The general form
+// divides in 64 bits, four times an index: 1000 instructions, which bound these
+// kernels.  Tiles of powers of two need shifts, and where a tile is whole
+// waves its position is the same in every lane, one scalar division per axis
+// (200^3 in 4x4x4 tiles: geometry of Riemann3 565 -> 150 us, expand 43 -> 21,
+// squeeze 40 -> 24; Riemann2 2000^2 143 -> 26).
+enum { kFormAny = 0, kFormShift = 1, kFormWave = 2 };
 
 static int make_layout(int32_t ndim, const int64_t* shape, const int32_t* shape_i, LayoutDesc& L) {
   AGD_REQUIRE(ndim >= 1 && ndim <= 3, "ndim must be 1..3");
@@ -54,11 +64,41 @@ static int make_layout(int32_t ndim, const int64_t* shape, const int32_t* shape_
     ntiles *= L.shape_o[k];
   }
   L.size_tot = ntiles * L.size_i;
+  auto log2_of = [](int32_t n) {
+    int l = 0;
+    while ((1 << l) < n) ++l;
+    return l;
+  };
+  bool pow2 = L.size_tot < (int64_t(1) << 31) && L.ncell < (int64_t(1) << 31);
+  for (int k = 0; k < 3; ++k) {
+    L.ls[k] = log2_of(L.shape_i[k]);
+    pow2 = pow2 && (1 << L.ls[k]) == L.shape_i[k];
+  }
+  L.lsize = log2_of(L.size_i);
+  L.form = !pow2 ? kFormAny : (L.size_i >= 64 ? kFormWave : kFormShift);
   return AGD_OK;
 }
 
 // Tiled index -> cell position (returns false in the padding).
+template <int FORM>
 __device__ inline bool tiled_to_cell(const LayoutDesc& L, int64_t n_t, int64_t& cell) {
+  if constexpr (FORM != kFormAny) {
+    uint32_t n_o = uint32_t(n_t) >> L.lsize;
+    if constexpr (FORM == kFormWave) n_o = __builtin_amdgcn_readfirstlane(n_o);
+    uint32_t n_i = uint32_t(n_t) & uint32_t(L.size_i - 1);
+    const uint32_t r = n_o / uint32_t(L.shape_o[2]), q = r / uint32_t(L.shape_o[1]);
+    const uint32_t xo[3] = {q, r - q * uint32_t(L.shape_o[1]), n_o - r * uint32_t(L.shape_o[2])};
+    uint32_t x[3];
+    bool in = true;
+#pragma unroll
+    for (int k = 2; k >= 0; --k) {
+      x[k] = (xo[k] << L.ls[k]) + (n_i & uint32_t(L.shape_i[k] - 1));
+      n_i >>= L.ls[k];
+      in = in && x[k] < uint32_t(L.shape[k]);
+    }
+    cell = (x[0] * uint32_t(L.shape[1]) + x[1]) * uint32_t(L.shape[2]) + x[2];
+    return in;
+  }
   int64_t n_o = n_t / L.size_i;
   int n_i = int(n_t - n_o * L.size_i);
   int xo[3], xi[3];
@@ -77,13 +117,13 @@ __device__ inline bool tiled_to_cell(const LayoutDesc& L, int64_t n_t, int64_t& 
   return true;
 }
 
-template <class T>
+template <class T, int FORM>
 __global__ void expand_kernel(LayoutDesc L, int32_t ncomp, const T* src, int64_t stride, T* dst,
                               T pad) {
   const int64_t n_t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (n_t >= L.size_tot) return;
   int64_t cell;
-  const bool in = tiled_to_cell(L, n_t, cell);
+  const bool in = tiled_to_cell<FORM>(L, n_t, cell);
   for (int c = 0; c < ncomp; ++c) {
     T v = pad;
     if (in) v = stride == 0 ? src[c] : src[c * L.ncell + cell];
@@ -91,18 +131,18 @@ __global__ void expand_kernel(LayoutDesc L, int32_t ncomp, const T* src, int64_t
   }
 }
 
-template <class T>
+template <class T, int FORM>
 __global__ void squeeze_kernel(LayoutDesc L, int32_t ncomp, const T* src, T* dst) {
   const int64_t n_t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (n_t >= L.size_tot) return;
   int64_t cell;
-  if (!tiled_to_cell(L, n_t, cell)) return;
+  if (!tiled_to_cell<FORM>(L, n_t, cell)) return;
   for (int c = 0; c < ncomp; ++c) dst[c * L.ncell + cell] = src[c * L.size_tot + n_t];
 }
 
 // Symmetric 2x2 / 3x3 inverse in double precision (cofactors).
-__device__ inline void inv_sym(int d, const double (&a)[3][3], double (&r)[3][3]) {
-  if (d == 2) {
+template <int D> __device__ inline void inv_sym(const double (&a)[3][3], double (&r)[3][3]) {
+  if constexpr (D == 2) {
     const double det = a[0][0] * a[1][1] - a[0][1] * a[1][0];
     r[0][0] = a[1][1] / det;
     r[1][1] = a[0][0] / det;
@@ -125,83 +165,129 @@ __device__ inline void inv_sym(int d, const double (&a)[3][3], double (&r)[3][3]
 }
 
 // General 2x2 / 3x3 inverse in double precision (adjugate / determinant).
-__device__ inline void inv_gen(int d, const double (&a)[3][3], double (&r)[3][3]) {
-  if (d == 2) {
+template <int D> __device__ inline void inv_gen(const double (&a)[3][3], double (&r)[3][3]) {
+  if constexpr (D == 2) {
     const double det = a[0][0] * a[1][1] - a[0][1] * a[1][0];
     r[0][0] = a[1][1] / det;
     r[0][1] = -a[0][1] / det;
     r[1][0] = -a[1][0] / det;
     r[1][1] = a[0][0] / det;
-    return;
+  } else {
+    double c[3][3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {
+        const int i1 = (i + 1) % 3, i2 = (i + 2) % 3, j1 = (j + 1) % 3, j2 = (j + 2) % 3;
+        c[i][j] = a[i1][j1] * a[i2][j2] - a[i1][j2] * a[i2][j1];  // cofactor (i, j)
+      }
+    const double det = a[0][0] * c[0][0] + a[0][1] * c[0][1] + a[0][2] * c[0][2];
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+      for (int j = 0; j < 3; ++j) r[i][j] = c[j][i] / det;
   }
-  double c[3][3];
-  for (int i = 0; i < 3; ++i)
-    for (int j = 0; j < 3; ++j) {
-      const int i1 = (i + 1) % 3, i2 = (i + 2) % 3, j1 = (j + 1) % 3, j2 = (j + 2) % 3;
-      c[i][j] = a[i1][j1] * a[i2][j2] - a[i1][j2] * a[i2][j1];  // cofactor (i, j)
-    }
-  const double det = a[0][0] * c[0][0] + a[0][1] * c[0][1] + a[0][2] * c[0][2];
-  for (int i = 0; i < 3; ++i)
-    for (int j = 0; j < 3; ++j) r[i][j] = c[j][i] / det;
 }
 
-template <class S>
-__global__ void geometry_kernel(LayoutDesc L, int32_t model, double h0, double h1, double h2,
-                                const float* m, const float* w, int64_t stride, S* geom) {
+// Bound by its bytes once the index arithmetic is scalar and the matrices stay
+// in registers (model and dimension are compile-time: indexed at run time, they
+// would live in scratch memory).
+template <class S, int MODEL, int D, int FORM>
+__global__ void __launch_bounds__(256) geometry_kernel(LayoutDesc L, double h0, double h1, double h2, const float* m,
+                                                       const float* w, int64_t stride, S* geom) {
   const int64_t n_t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (n_t >= L.size_tot) return;
-  const int d = L.ndim;
   const double h[3] = {h0, h1, h2};
-  const int sd = d * (d + 1) / 2;
+  constexpr int SD = D * (D + 1) / 2;
+  constexpr int NG = MODEL == AGD_DIAGONAL ? D : MODEL == AGD_TTI ? 5 + D * D : MODEL == AGD_RANDER ? SD + D : SD;
   int64_t cell;
-  const bool in = tiled_to_cell(L, n_t, cell);
+  const bool in = tiled_to_cell<FORM>(L, n_t, cell);
   const int64_t c = stride == 0 ? 0 : cell;
   const int64_t cs = stride == 0 ? 1 : L.ncell;  // component stride of the source
-  if (model == AGD_DIAGONAL) {
-    for (int k = 0; k < d; ++k) {
-      double v = inf_v<double>();
-      if (in) {
-        const double ch = double(m[k * cs + c]) * h[k];
-        v = 1.0 / (ch * ch);
-      }
-      geom[k * L.size_tot + n_t] = S(v);
-    }
+  if (!in) {
+#pragma unroll
+    for (int k = 0; k < NG; ++k) geom[k * L.size_tot + n_t] = inf_v<S>();
     return;
   }
-  if (model == AGD_TTI) {
+  if constexpr (MODEL == AGD_DIAGONAL) {
+#pragma unroll
+    for (int k = 0; k < D; ++k) {
+      const double ch = double(m[k * cs + c]) * h[k];
+      geom[k * L.size_tot + n_t] = S(1.0 / (ch * ch));
+    }
+  } else if constexpr (MODEL == AGD_TTI) {
     // TTI.with_costs(h).flatten(transposed_transformation=True)
     // (Seismic/tti.py:113-125, Metrics/base.py:175-185): [l, flat(q),
     // (A diag(h))^{-T}], A = w (row-major, identity if null).
-    const int ng = 5 + d * d;
-    if (!in) {
-      for (int k = 0; k < ng; ++k) geom[k * L.size_tot + n_t] = inf_v<S>();
-      return;
-    }
+#pragma unroll
     for (int k = 0; k < 5; ++k) geom[k * L.size_tot + n_t] = S(double(m[k * cs + c]));
     double A[3][3], r[3][3];
-    for (int i = 0; i < d; ++i)
-      for (int j = 0; j < d; ++j)
-        A[i][j] = (w ? double(w[(i * d + j) * cs + c]) : double(i == j)) * h[j];
-    inv_gen(d, A, r);
-    for (int i = 0; i < d; ++i)
-      for (int j = 0; j < d; ++j) geom[(5 + i * d + j) * L.size_tot + n_t] = S(r[j][i]);
-    return;
+#pragma unroll
+    for (int i = 0; i < D; ++i)
+#pragma unroll
+      for (int j = 0; j < D; ++j) A[i][j] = (w ? double(w[(i * D + j) * cs + c]) : double(i == j)) * h[j];
+    inv_gen<D>(A, r);
+#pragma unroll
+    for (int i = 0; i < D; ++i)
+#pragma unroll
+      for (int j = 0; j < D; ++j) geom[(5 + i * D + j) * L.size_tot + n_t] = S(r[j][i]);
+  } else {
+    double a[3][3], r[3][3];
+#pragma unroll
+    for (int i = 0; i < D; ++i)
+#pragma unroll
+      for (int j = 0; j < D; ++j) a[i][j] = double(m[(i * D + j) * cs + c]) * h[i] * h[j];
+    inv_sym<D>(a, r);
+    int k = 0;
+#pragma unroll
+    for (int i = 0; i < D; ++i)
+#pragma unroll
+      for (int j = 0; j <= i; ++j, ++k) geom[k * L.size_tot + n_t] = S(r[i][j]);
+    if constexpr (MODEL == AGD_RANDER) {
+#pragma unroll
+      for (int i = 0; i < D; ++i) geom[(SD + i) * L.size_tot + n_t] = S(double(w[i * cs + c]) * h[i]);
+    }
   }
-  const int ng = model == AGD_RANDER ? sd + d : sd;
-  if (!in) {
-    for (int k = 0; k < ng; ++k) geom[k * L.size_tot + n_t] = inf_v<S>();
-    return;
+}
+
+template <class S, int MODEL, int D>
+static void launch_geometry(const LayoutDesc& L, const double* h, const float* m, const float* w, int64_t stride,
+                            S* geom, hipStream_t s) {
+  const dim3 grid(unsigned(ceil_div(L.size_tot, 256))), block(256);
+  auto kern = L.form == kFormWave    ? geometry_kernel<S, MODEL, D, kFormWave>
+              : L.form == kFormShift ? geometry_kernel<S, MODEL, D, kFormShift>
+                                     : geometry_kernel<S, MODEL, D, kFormAny>;
+  hipLaunchKernelGGL(kern, grid, block, 0, s, L, h[0], h[1], D == 3 ? h[2] : 1.0, m, w, stride, geom);
+}
+
+template <class S, int D>
+static void launch_geometry_model(int model, const LayoutDesc& L, const double* h, const float* m, const float* w,
+                                  int64_t stride, S* geom, hipStream_t s) {
+  switch (model) {
+    case AGD_DIAGONAL: return launch_geometry<S, AGD_DIAGONAL, D>(L, h, m, w, stride, geom, s);
+    case AGD_RIEMANN: return launch_geometry<S, AGD_RIEMANN, D>(L, h, m, w, stride, geom, s);
+    case AGD_RANDER: return launch_geometry<S, AGD_RANDER, D>(L, h, m, w, stride, geom, s);
+    case AGD_TTI: return launch_geometry<S, AGD_TTI, D>(L, h, m, w, stride, geom, s);
   }
-  double a[3][3], r[3][3];
-  for (int i = 0; i < d; ++i)
-    for (int j = 0; j < d; ++j) a[i][j] = double(m[(i * d + j) * cs + c]) * h[i] * h[j];
-  inv_sym(d, a, r);
-  int k = 0;
-  for (int i = 0; i < d; ++i)
-    for (int j = 0; j <= i; ++j, ++k) geom[k * L.size_tot + n_t] = S(r[i][j]);
-  if (model == AGD_RANDER) {
-    for (int i = 0; i < d; ++i) geom[(sd + i) * L.size_tot + n_t] = S(double(w[i * cs + c]) * h[i]);
-  }
+}
+
+template <class T>
+static void launch_expand(const LayoutDesc& L, int32_t ncomp, const void* src, int64_t stride, void* dst, T pad,
+                          hipStream_t s) {
+  const dim3 grid(unsigned(ceil_div(L.size_tot, 256))), block(256);
+  auto kern = L.form == kFormWave    ? expand_kernel<T, kFormWave>
+              : L.form == kFormShift ? expand_kernel<T, kFormShift>
+                                     : expand_kernel<T, kFormAny>;
+  hipLaunchKernelGGL(kern, grid, block, 0, s, L, ncomp, static_cast<const T*>(src), stride, static_cast<T*>(dst), pad);
+}
+
+template <class T>
+static void launch_squeeze(const LayoutDesc& L, int32_t ncomp, const void* src, void* dst, hipStream_t s) {
+  const dim3 grid(unsigned(ceil_div(L.size_tot, 256))), block(256);
+  auto kern = L.form == kFormWave    ? squeeze_kernel<T, kFormWave>
+              : L.form == kFormShift ? squeeze_kernel<T, kFormShift>
+                                     : squeeze_kernel<T, kFormAny>;
+  hipLaunchKernelGGL(kern, grid, block, 0, s, L, ncomp, static_cast<const T*>(src), static_cast<T*>(dst));
 }
 
 }  // namespace agd
@@ -228,24 +314,11 @@ int agd_block_expand(int32_t ndim, const int64_t* shape, const int32_t* shape_i,
   if (st) return st;
   AGD_REQUIRE(src && dst && ncomp >= 1, "bad buffers");
   AGD_REQUIRE(src_cell_stride == 0 || src_cell_stride == 1, "cell stride must be 0 or 1");
-  const dim3 grid(unsigned(ceil_div(L.size_tot, 256))), block(256);
   hipStream_t s = as_stream(stream);
   switch (elem_size) {
-    case 1:
-      hipLaunchKernelGGL(expand_kernel<uint8_t>, grid, block, 0, s, L, ncomp,
-                         static_cast<const uint8_t*>(src), src_cell_stride,
-                         static_cast<uint8_t*>(dst), uint8_t(pad));
-      break;
-    case 4:
-      hipLaunchKernelGGL(expand_kernel<float>, grid, block, 0, s, L, ncomp,
-                         static_cast<const float*>(src), src_cell_stride,
-                         static_cast<float*>(dst), float(pad));
-      break;
-    case 8:
-      hipLaunchKernelGGL(expand_kernel<double>, grid, block, 0, s, L, ncomp,
-                         static_cast<const double*>(src), src_cell_stride,
-                         static_cast<double*>(dst), pad);
-      break;
+    case 1: launch_expand<uint8_t>(L, ncomp, src, src_cell_stride, dst, uint8_t(pad), s); break;
+    case 4: launch_expand<float>(L, ncomp, src, src_cell_stride, dst, float(pad), s); break;
+    case 8: launch_expand<double>(L, ncomp, src, src_cell_stride, dst, pad, s); break;
     default: set_error("invalid argument: elem_size must be 1, 4 or 8"); return AGD_EINVAL;
   }
   AGD_HIP_TRY(hipGetLastError());
@@ -258,21 +331,11 @@ int agd_block_squeeze(int32_t ndim, const int64_t* shape, const int32_t* shape_i
   int st = make_layout(ndim, shape, shape_i, L);
   if (st) return st;
   AGD_REQUIRE(src && dst && ncomp >= 1, "bad buffers");
-  const dim3 grid(unsigned(ceil_div(L.size_tot, 256))), block(256);
   hipStream_t s = as_stream(stream);
   switch (elem_size) {
-    case 1:
-      hipLaunchKernelGGL(squeeze_kernel<uint8_t>, grid, block, 0, s, L, ncomp,
-                         static_cast<const uint8_t*>(src), static_cast<uint8_t*>(dst));
-      break;
-    case 4:
-      hipLaunchKernelGGL(squeeze_kernel<float>, grid, block, 0, s, L, ncomp,
-                         static_cast<const float*>(src), static_cast<float*>(dst));
-      break;
-    case 8:
-      hipLaunchKernelGGL(squeeze_kernel<double>, grid, block, 0, s, L, ncomp,
-                         static_cast<const double*>(src), static_cast<double*>(dst));
-      break;
+    case 1: launch_squeeze<uint8_t>(L, ncomp, src, dst, s); break;
+    case 4: launch_squeeze<float>(L, ncomp, src, dst, s); break;
+    case 8: launch_squeeze<double>(L, ncomp, src, dst, s); break;
     default: set_error("invalid argument: elem_size must be 1, 4 or 8"); return AGD_EINVAL;
   }
   AGD_HIP_TRY(hipGetLastError());
@@ -292,15 +355,14 @@ int agd_prepare_geometry(int32_t model, int32_t ndim, const int64_t* shape, cons
   AGD_REQUIRE(h && m && geom, "null buffer");
   AGD_REQUIRE(model != AGD_RANDER || w, "Rander model needs the drift w");
   AGD_REQUIRE(cell_stride == 0 || cell_stride == 1, "cell stride must be 0 or 1");
-  const dim3 grid(unsigned(ceil_div(L.size_tot, 256))), block(256);
   hipStream_t s = as_stream(stream);
-  const double h2 = ndim == 3 ? h[2] : 1.0;
-  if (scalar == AGD_F32)
-    hipLaunchKernelGGL(geometry_kernel<float>, grid, block, 0, s, L, model, h[0], h[1], h2, m, w,
-                       cell_stride, static_cast<float*>(geom));
-  else
-    hipLaunchKernelGGL(geometry_kernel<double>, grid, block, 0, s, L, model, h[0], h[1], h2, m, w,
-                       cell_stride, static_cast<double*>(geom));
+  if (scalar == AGD_F32) {
+    if (ndim == 2) launch_geometry_model<float, 2>(model, L, h, m, w, cell_stride, static_cast<float*>(geom), s);
+    else launch_geometry_model<float, 3>(model, L, h, m, w, cell_stride, static_cast<float*>(geom), s);
+  } else {
+    if (ndim == 2) launch_geometry_model<double, 2>(model, L, h, m, w, cell_stride, static_cast<double*>(geom), s);
+    else launch_geometry_model<double, 3>(model, L, h, m, w, cell_stride, static_cast<double*>(geom), s);
+  }
   AGD_HIP_TRY(hipGetLastError());
   return AGD_OK;
 }
