@@ -329,9 +329,17 @@ class Interface:
             # a physical (nx, ny) or angular (ntheta) cost field is broadcast
             # over the grid (_Interface.py:221-234); the curvature schemes are
             # in units of the physical cell side h (_SetGeometry.py:234)
-            if np.ndim(host_array(self.cost)) > 0:
-                self.cost = np.ascontiguousarray(self._angular_field(self.cost, 'cost'))
-            self.cost = self.cost * self.curvature_cost_scale
+            # (cost_part: what was given, scaled; it is spread on the device)
+            if isinstance(self.cost, torch.Tensor):
+                part = self.cost.detach().double()
+                part = part.reshape(self._angular_axes(tuple(part.shape), 'cost')) if part.dim() else part
+                self.cost_part = part * self.curvature_cost_scale
+                self.cost = self.cost_part.expand(tuple(self.shape)) if part.dim() else self.cost_part
+            elif np.ndim(host_array(self.cost)) > 0:
+                self.cost_part = self._angular_part(self.cost, 'cost') * self.curvature_cost_scale
+                self.cost = np.broadcast_to(self.cost_part, tuple(self.shape))
+            else:
+                self.cost = self.cost_part = self.cost * self.curvature_cost_scale
             if self.cost_coef is not None:
                 self.cost_coef = self.cost_coef * self.curvature_cost_scale
 
@@ -343,9 +351,9 @@ class Interface:
             tol = self.GetValue('tol', default="_Dummy",
                                 help="Convergence tolerance for the fixed point solver (determines atol, rtol)")
             if isinstance(tol, str) and tol == "_Dummy":
-                c = self.cost
-                mean_cost = float(torch.nanmean(c.float()).item()) if hasattr(c, 'detach') \
-                    else float(np.nanmean(np.asarray(c, dtype=np.float64)))
+                c = self.cost_part if self.curvature else self.cost
+                mean_cost = float(torch.nanmean(c if c.dtype == torch.float64 else c.float()).item()) \
+                    if hasattr(c, 'detach') else float(np.nanmean(np.asarray(c, dtype=np.float64)))
                 tol = mean_cost * res * 5.
                 self.hfmOut['keys']['default']['tol'] = self.tol_float_t(tol)
         self.atol = float(self.GetValue('atol', default=tol,
@@ -366,18 +374,27 @@ class Interface:
                 'minChg_delta_min', default=float(np.min(self.h)) / 10.,
                 help="Minimal threshold increase with bound_active_blocks method"))
 
-    def _angular_field(self, value, name):
-        """A scalar, a physical field (nx, ny), an angular field (ntheta) or a
-        full field, broadcast to the (x, y, theta) grid (_Interface.py:221-236)."""
+    def _angular_axes(self, shape, name):
+        """Three-axis shape of a scalar, a physical field (nx, ny), an angular
+        field (ntheta) or a full field: 1 along the axes that it is broadcast
+        over (_Interface.py:221-236)."""
+        full = tuple(self.shape)
+        if shape == ():
+            return (1, 1, 1)
+        if shape == full:
+            return full
+        if shape == full[2:]:
+            return (1, 1) + full[2:]
+        if shape == full[:2]:
+            return full[:2] + (1,)
+        raise ValueError(f"Field {name} has incorrect dimensions {shape} for the grid {full}")
+
+    def _angular_part(self, value, name):
         a = np.asarray(host_array(value), dtype=np.float64)
-        shape = tuple(self.shape)
-        if a.ndim == 0 or a.shape == shape:
-            return np.broadcast_to(a, shape)
-        if a.shape == shape[2:]:
-            return np.broadcast_to(a.reshape((1, 1) + shape[2:]), shape)
-        if a.shape == shape[:2]:
-            return np.broadcast_to(a.reshape(shape[:2] + (1,)), shape)
-        raise ValueError(f"Field {name} has incorrect dimensions {a.shape} for the grid {shape}")
+        return a.reshape(self._angular_axes(a.shape, name))
+
+    def _angular_field(self, value, name):
+        return np.broadcast_to(self._angular_part(value, name), tuple(self.shape))
 
     def _set_curvature_geometry(self):
         """Curvature models (_SetGeometry.py:83-109, _Kernel.py:318-332): per
@@ -396,21 +413,25 @@ class Interface:
         if not eps > 0:
             raise ValueError("eps must be > 0")
         self.curvature_relax = eps * eps
-        ixi = 1. / (self._angular_field(xi, 'xi') * ratio)
-        kap = self._angular_field(kappa, 'kappa') / ratio
+        ixi = 1. / (self._angular_part(xi, 'xi') * ratio)
+        kap = self._angular_part(kappa, 'kappa') / ratio
         if np.ndim(host_array(theta)) == 0:
             # a scalar theta selects the angles of the grid's third axis
-            th = self._angular_field(np.asarray(host_array(self.hfmIn.Axes()[2]), dtype=np.float64), 'theta')
+            th = self._angular_part(np.asarray(host_array(self.hfmIn.Axes()[2]), dtype=np.float64), 'theta')
         else:
-            th = self._angular_field(theta, 'theta')
-        geom = np.stack([ixi, kap, np.cos(th), np.sin(th)])
-        g_d = device_tensor(np.ascontiguousarray(geom), self.float_t)
+            th = self._angular_part(theta, 'theta')
+        # spread over the grid on the device
+        parts = [ixi, kap, np.cos(th), np.sin(th)]
+        offset = np.concatenate([[0], np.cumsum([p.size for p in parts])])[:4]
+        stride = [[s // p.itemsize if n > 1 else 0 for s, n in zip(p.strides, p.shape)]
+                  for p in map(np.ascontiguousarray, parts)]
+        src_d = device_tensor(np.concatenate([p.reshape(-1) for p in parts]), np.float64)
         self.geom = empty((4, self.size_tot), self.float_t)
-        esize = np.dtype(self.float_t).itemsize
-        _lib.check(_lib.lib.agd_block_expand(self.ndim, _lib.i64(self.shape), _lib.i32(self.shape_i), 4,
-                                             esize, ptr(g_d), 1, ptr(self.geom),
-                                             0., self.stream))
-        self._keep = (g_d,)
+        _lib.check(_lib.lib.agd_spread_fields(
+            self.ndim, _lib.i64(self.shape), _lib.i32(self.shape_i), 4, self.scalar, ptr(src_d),
+            (ctypes.c_int64 * 4)(*offset.tolist()), (ctypes.c_int64 * 12)(*sum(stride, [])), ptr(self.geom),
+            0., self.stream))
+        self._keep = (src_d,)
         self.curvature_cost_scale = h_base
 
     def _set_metric_geometry(self, metric, dualMetric):
@@ -542,7 +563,10 @@ class Interface:
             help="Start with every tile active (use with an initial supersolution 'values')"))
 
         # rhs = cost, padded with +inf
-        cost = device_tensor(self.cost, self.float_t)
+        if self.curvature and len(np.shape(self.cost_part)) > 0:
+            cost = device_tensor(self.cost_part, self.float_t).expand(tuple(self.shape)).contiguous()
+        else:
+            cost = device_tensor(self.cost, self.float_t)
         self.rhs_t = empty((self.size_tot,), self.float_t)
         if cost.dim() == 0:
             stride = 0

@@ -417,7 +417,13 @@ int agd_chart_paste(const agd_eikonal_desc* desc, void* values, const void* mapp
 int agd_block_expand(int32_t ndim, const int64_t* shape, const int32_t* shape_i,
                      int32_t ncomp, int32_t elem_size, const void* src,
                      int64_t src_cell_stride, void* dst, double pad, void* stream);
-/* block_squeeze (FiniteDifferences.py:197-222): inverse of the above. */
+/* Fields given on a part of the axes, spread over the tiled grid: component c
+ * (at most 8) of cell x is src[offset[c] + sum_k x_k stride[c * ndim + k]],
+ * strides >= 0 (0: the same along the axis), rounded to `scalar`. */
+int agd_spread_fields(int32_t ndim, const int64_t* shape, const int32_t* shape_i, int32_t ncomp,
+                      int32_t scalar, const double* src, const int64_t* offset, const int64_t* stride,
+                      void* dst, double pad, void* stream);
+/* block_squeeze (FiniteDifferences.py:197-222): inverse of agd_block_expand. */
 int agd_block_squeeze(int32_t ndim, const int64_t* shape, const int32_t* shape_i,
                       int32_t ncomp, int32_t elem_size, const void* src, void* dst,
                       void* stream);

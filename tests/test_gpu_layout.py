@@ -67,3 +67,30 @@ def test_riemann_geometry(shape, tile, const):
     pad = np.ones(size, bool)
     pad[idx] = False
     assert np.all(np.isinf(g[:, pad]))
+
+
+@pytest.mark.parametrize("tile", [(4, 4, 4), (3, 4, 5)])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_spread_fields(tile, dtype):
+    """A constant, a plane, a line and a full field, spread and rounded exactly."""
+    import ctypes
+    import torch
+    shape = (5, 9, 6)
+    log(f"spread {shape} in {tile} {np.dtype(dtype).name}")
+    rng = np.random.default_rng(2)
+    parts = [rng.normal(size=s) for s in ((1, 1, 1), (5, 9, 1), (1, 1, 6), shape)]
+    so = fd.round_up_ratio(shape, tile)
+    size = int(np.prod(so) * np.prod(tile))
+    idx = fd.tiled_index(np.stack(np.meshgrid(*map(np.arange, shape), indexing='ij'), -1), tile, so)
+    ref = np.full((4, size), -1, dtype)
+    for c, p in enumerate(parts):
+        ref[c][idx] = np.broadcast_to(p, shape).astype(dtype)
+    src = torch.from_numpy(np.concatenate([p.reshape(-1) for p in parts])).cuda()
+    offset = np.concatenate([[0], np.cumsum([p.size for p in parts])])[:4].tolist()
+    stride = sum([[s // 8 if n > 1 else 0 for s, n in zip(p.strides, p.shape)] for p in parts], [])
+    out = torch.empty((4, size), dtype=torch.float32 if dtype == np.float32 else torch.float64, device='cuda')
+    _lib.check(_lib.lib.agd_spread_fields(
+        3, _lib.i64(shape), _lib.i32(tile), 4, _lib.F32 if dtype == np.float32 else _lib.F64, src.data_ptr(),
+        (ctypes.c_int64 * 4)(*offset), (ctypes.c_int64 * 12)(*stride), out.data_ptr(), -1., None))
+    torch.cuda.synchronize()
+    assert np.array_equal(out.cpu().numpy(), ref)
