@@ -730,10 +730,10 @@ class Interface:
                                                    help="Raise an exception if a solver fails to converge")
         self.check_interval = int(self.GetValue(
             'check_interval', default=18,
-            help="Grid passes between two convergence checks on the host"))
+            help="Grid passes between two convergence checks on the host (hipGraph False)"))
         self.use_graph = bool(self.GetValue(
             'hipGraph', default=True,
-            help="Capture check_interval grid passes once as a hipGraph and replay it"))
+            help="Queue grid passes ahead of the device, without waiting every check_interval passes"))
 
     def _desc(self, niter_i=None):
         d = _lib.EikonalDesc()

@@ -90,6 +90,7 @@ SIGNATURES = {
     "agd_batch_tile_supported": (c_int32, [c_int32, c_int32, c_int32_p]),
     "agd_device_count": (c_int32, [c_int32_p]),
     "agd_solver_create": (c_int32, [POINTER(EikonalDesc), c_void_p, POINTER(c_void_p)]),
+    "agd_release_workspaces": (c_int32, [c_int64_p]),
     "agd_solver_destroy": (c_int32, [c_void_p]),
     "agd_solver_solve": (c_int32, [c_void_p, POINTER(EikonalDesc), POINTER(EikonalIO),
                                    POINTER(EikonalStats)]),
@@ -234,6 +235,13 @@ def i64(seq):
 def i32(seq):
     arr = (c_int32 * 3)(*([int(s) for s in seq] + [1] * (3 - len(seq))))
     return arr
+
+
+def release_workspaces():
+    """Free the idle workspaces kept on the current device; their bytes."""
+    n = c_int64(0)
+    check(lib.agd_release_workspaces(ctypes.byref(n)))
+    return int(n.value)
 
 
 class Solver:

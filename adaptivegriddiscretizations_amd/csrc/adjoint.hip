@@ -298,30 +298,36 @@ static int linear_impl(bool forward, const agd_eikonal_desc* d, const S* values,
   const int nsym = nsym_of(d->model, d->ndim);
   const dim3 grid(unsigned(ceil_div(N, 256))), block(256);
 
-  // ---- 1. the system's rows (reverse: transposed flow graph)
-  int32_t *deg = nullptr, *rowptr = nullptr, *rowloc = nullptr, *src = nullptr;
-  uint32_t* trig = nullptr;
-  S* wt = nullptr;
-  void* tmp = nullptr;
+  // ---- 1. the system's rows (reverse: transposed flow graph), in the
+  // workspace: [deg, trig (cleared)], rowptr, rowloc, the scan's own
+  WorkspaceLease lease;
+  Workspace& ws = *lease;
   size_t tmp_bytes = 0;
-  AGD_HIP_TRY(hipMalloc((void**)&deg, (N + 1) * sizeof(int32_t)));
-  AGD_HIP_TRY(hipMalloc((void**)&rowptr, (N + 1) * sizeof(int32_t)));
-  AGD_HIP_TRY(hipMalloc((void**)&rowloc, N * sizeof(int32_t)));
-  AGD_HIP_TRY(hipMalloc((void**)&trig, ceil_div(N, 32) * sizeof(uint32_t)));
-  AGD_HIP_TRY(hipMemsetAsync(deg, 0, (N + 1) * sizeof(int32_t), stream));
-  AGD_HIP_TRY(hipMemsetAsync(trig, 0, ceil_div(N, 32) * sizeof(uint32_t), stream));
+  AGD_HIP_TRY(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp_bytes, static_cast<int32_t*>(nullptr),
+                                               static_cast<int32_t*>(nullptr), int(N + 1), stream));
+  auto up = [](size_t b) { return (b + 255) & ~size_t(255); };
+  const size_t b_deg = up(size_t(N + 1) * 4), b_trig = up(size_t(ceil_div(N, 32)) * 4), b_loc = up(size_t(N) * 4);
+  if (int st = ws.ensure_scratch(2 * b_deg + b_trig + b_loc + tmp_bytes)) return st;
+  ws.busy = true;
+  char* const base = static_cast<char*>(ws.scratch);
+  int32_t* const deg = reinterpret_cast<int32_t*>(base);
+  uint32_t* const trig = reinterpret_cast<uint32_t*>(base + b_deg);
+  int32_t* const rowptr = reinterpret_cast<int32_t*>(base + b_deg + b_trig);
+  int32_t* const rowloc = reinterpret_cast<int32_t*>(base + 2 * b_deg + b_trig);
+  void* const tmp = base + 2 * b_deg + b_trig + b_loc;
+  fill_i32(deg, int64_t((b_deg + b_trig) / 4), 0, stream);
   if (forward)
     hipLaunchKernelGGL(fwd_count<S>, grid, block, 0, stream, N, nsym, fw, fidx, deg);
   else
     hipLaunchKernelGGL(adj_count<S>, grid, block, 0, stream, N, nsym, fw, fidx, deg);
-  AGD_HIP_TRY(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp_bytes, deg, rowptr, int(N + 1), stream));
-  AGD_HIP_TRY(hipMalloc(&tmp, tmp_bytes));
   AGD_HIP_TRY(hipcub::DeviceScan::ExclusiveSum(tmp, tmp_bytes, deg, rowptr, int(N + 1), stream));
   int32_t nnz = 0;
   AGD_HIP_TRY(hipMemcpyAsync(&nnz, rowptr + N, sizeof(int32_t), hipMemcpyDeviceToHost, stream));
   AGD_HIP_TRY(hipStreamSynchronize(stream));
-  AGD_HIP_TRY(hipMalloc((void**)&src, std::max<int64_t>(nnz, 1) * sizeof(int32_t)));
-  AGD_HIP_TRY(hipMalloc((void**)&wt, std::max<int64_t>(nnz, 1) * sizeof(S)));
+  const size_t b_src = up(size_t(std::max<int64_t>(nnz, 1)) * 4);
+  if (int st = ws.ensure_region(b_src + size_t(std::max<int64_t>(nnz, 1)) * sizeof(S))) return st;
+  int32_t* const src = static_cast<int32_t*>(ws.region);
+  S* const wt = reinterpret_cast<S*>(static_cast<char*>(ws.region) + b_src);
   if (forward) {
     hipLaunchKernelGGL(fwd_fill<S>, grid, block, 0, stream, N, nsym, fw, fidx, rowptr, src, wt);
   } else {
@@ -336,7 +342,6 @@ static int linear_impl(bool forward, const agd_eikonal_desc* d, const S* values,
 
   // ---- 2. tile Gauss-Seidel, one right-hand side at a time
   const int blocks = blocks_for(g.ntiles, ls.ni);
-  Workspace ws;  // this call's own worklist, released on return
   int64_t niter = 0, visits = 0, passes = 0;
   float ms = 0.f;
   double kernel_ms = 0.;
@@ -344,7 +349,7 @@ static int linear_impl(bool forward, const agd_eikonal_desc* d, const S* values,
   int status = AGD_OK;
   for (int r = 0; r < nrhs && status == AGD_OK; ++r) {
     LinArgs<S> a;
-    std::memset(&a, 0, sizeof a);  // zeroed padding: the bytes key the graph cache
+    std::memset(&a, 0, sizeof a);
     a.lam = lam + int64_t(r) * N;
     a.rhs = sens + int64_t(r) * N;
     a.diag = wsum;
@@ -371,18 +376,13 @@ static int linear_impl(bool forward, const agd_eikonal_desc* d, const S* values,
                          trig, g.ntiles, ws->stamp, ws->lists, ws->counts, a.w.shard_cap);
       return AGD_OK;
     };
-    auto launch = [&](int32_t koff, hipStream_t s, bool phase) {
+    auto launch = [&](int32_t koff, hipStream_t s) {
       a.w.koff = koff;
-      a.w.phase_from_koff = phase ? 1 : 0;
       hipLaunchKernelGGL(ls.update, dim3(blocks), dim3(ls.ni), 0, s, a);
-    };
-    auto key = [&](std::vector<unsigned char>& k) {
-      key_append(k, ls.update);
-      key_append(k, a);
     };
     WorklistResult res;
     status = run_worklist(ws, g.ntiles, blocks, d->nitermax_o, d->check_interval, stream, init,
-                          launch, key, res, d->time_launches != 0, d->use_graph != 0);
+                          launch, res, d->time_launches != 0, d->use_graph != 0);
     kernel_ms += res.kernel_ms;
     niter += res.niter;
     visits += res.visits;
@@ -390,14 +390,6 @@ static int linear_impl(bool forward, const agd_eikonal_desc* d, const S* values,
     ms += res.ms;
     converged = converged && res.converged;
   }
-  (void)hipStreamSynchronize(stream);
-  (void)hipFree(deg);
-  (void)hipFree(rowptr);
-  (void)hipFree(rowloc);
-  (void)hipFree(trig);
-  (void)hipFree(src);
-  (void)hipFree(wt);
-  (void)hipFree(tmp);
   if (status) return status;
   if (stats) {
     stats->niter_o = niter;

@@ -416,34 +416,31 @@ void Workspace::release() {
   if (!fixed) {
     free_dev(ftab);
     free_dev(region);
+    free_dev(scratch);
     free_dev(stamp);
     free_dev(needs);
     free_dev(pending);
     free_dev(bab);
     free_dev(lists);
     free_dev(counts);
-    free_dev(hist);
+    if (hist) (void)hipHostFree(hist);
     free_dev(score);
     free_dev(check_count);
     free_dev(inst);
     free_dev(tile_inst);
     if (host_counts) (void)hipHostFree(host_counts);
-    if (exec) (void)hipGraphExecDestroy(exec);
-    for (hipEvent_t e : {ev0, ev1, chunk_ev[0], chunk_ev[1]})
+    for (hipEvent_t e : {ev0, ev1})
       if (e) (void)hipEventDestroy(e);
-    if (capture_stream) (void)hipStreamDestroy(capture_stream);
   }
   stamp = needs = bab = lists = counts = hist = score = check_count = tile_inst = nullptr;
   pending = nullptr;
   inst = nullptr;
   host_counts = nullptr;
-  exec = nullptr;
-  exec_key.clear();
-  ev0 = ev1 = chunk_ev[0] = chunk_ev[1] = nullptr;
-  capture_stream = nullptr;
+  ev0 = ev1 = nullptr;
   tile_cap = shard_cap = hist_cap = inst_cap = tinst_cap = 0;
-  ftab = region = nullptr;
-  ftab_bytes = region_bytes = 0;
+  ftab = region = scratch = nullptr;
+  ftab_bytes = region_bytes = scratch_bytes = 0;
+  busy = false;
   fixed = false;
 }
 
@@ -468,6 +465,22 @@ int Workspace::ensure_region(size_t bytes) {
   return AGD_OK;
 }
 
+int Workspace::ensure_scratch(size_t bytes) {
+  AGD_REQUIRE(!fixed, "linear systems need an allocating workspace");
+  if (scratch_bytes < bytes) {
+    free_dev(scratch);
+    scratch_bytes = 0;
+    AGD_HIP_TRY(hipMalloc(&scratch, bytes));
+    scratch_bytes = bytes;
+  }
+  return AGD_OK;
+}
+
+size_t Workspace::bytes() const {
+  return ftab_bytes + region_bytes + scratch_bytes + size_t(tile_cap) * 24 + size_t(2 * kShards) * size_t(shard_cap) * 4 +
+         size_t(tinst_cap) * 4;
+}
+
 int Workspace::ensure(int64_t ntiles, int64_t scap, int64_t nhist) {
   if (fixed) {
     AGD_REQUIRE(ntiles <= tile_cap && scap <= shard_cap && nhist <= hist_cap,
@@ -477,10 +490,7 @@ int Workspace::ensure(int64_t ntiles, int64_t scap, int64_t nhist) {
   if (!ev0) {
     AGD_HIP_TRY(hipEventCreate(&ev0));
     AGD_HIP_TRY(hipEventCreate(&ev1));
-    AGD_HIP_TRY(hipHostMalloc((void**)&host_counts, 2 * kRow * sizeof(int32_t), hipHostMallocDefault));
-    AGD_HIP_TRY(hipEventCreateWithFlags(&chunk_ev[0], hipEventDisableTiming));
-    AGD_HIP_TRY(hipEventCreateWithFlags(&chunk_ev[1], hipEventDisableTiming));
-    AGD_HIP_TRY(hipStreamCreateWithFlags(&capture_stream, hipStreamNonBlocking));
+    AGD_HIP_TRY(hipHostMalloc((void**)&host_counts, kRow * sizeof(int32_t), hipHostMallocDefault));
     AGD_HIP_TRY(hipMalloc((void**)&counts, kCountsAlloc * sizeof(int32_t)));
     AGD_HIP_TRY(hipMalloc((void**)&check_count, 64));
     AGD_HIP_TRY(hipMalloc((void**)&bab, kBabLen * sizeof(int32_t)));
@@ -504,9 +514,11 @@ int Workspace::ensure(int64_t ntiles, int64_t scap, int64_t nhist) {
     shard_cap = cap;
   }
   if (hist_cap < nhist) {
-    free_dev(hist);
+    if (hist) (void)hipHostFree(hist);
+    hist = nullptr;
+    hist_cap = 0;
     const int64_t cap = std::max<int64_t>(nhist, 4096);
-    AGD_HIP_TRY(hipMalloc((void**)&hist, cap * sizeof(int32_t)));
+    AGD_HIP_TRY(hipHostMalloc((void**)&hist, cap * sizeof(int32_t), hipHostMallocDefault));
     hist_cap = cap;
   }
   return AGD_OK;
@@ -564,6 +576,47 @@ int Workspace::bind_fixed(void* base, size_t bytes, int64_t ntiles, int64_t scap
   return AGD_OK;
 }
 
+// ------------------------------------------------------------------ pool
+// Idle workspaces, per device.  Never destroyed: the HIP runtime may be gone
+// when static objects are.
+struct WorkspacePool {
+  std::mutex mutex;
+  std::vector<Workspace*> idle;
+};
+constexpr int kMaxDevices = 64;
+static WorkspacePool& pool_of(int device) {
+  static WorkspacePool* const pools = new WorkspacePool[kMaxDevices];
+  return pools[device];
+}
+
+WorkspaceLease::WorkspaceLease() : ws_(nullptr) {
+  int dev = 0;
+  if (hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < kMaxDevices) {
+    device_ = dev;
+    WorkspacePool& p = pool_of(dev);
+    std::lock_guard<std::mutex> lock(p.mutex);
+    if (!p.idle.empty()) {
+      ws_ = p.idle.back();
+      p.idle.pop_back();
+    }
+  }
+  if (!ws_) ws_ = new Workspace;
+}
+
+WorkspaceLease::~WorkspaceLease() {
+  if (device_ >= 0 && !ws_->busy) {
+    WorkspacePool& p = pool_of(device_);
+    std::lock_guard<std::mutex> lock(p.mutex);
+    size_t held = ws_->bytes();
+    for (const Workspace* w : p.idle) held += w->bytes();
+    if (p.idle.size() < kPoolMost && held <= kPoolBytes) {
+      p.idle.push_back(ws_);
+      return;
+    }
+  }
+  delete ws_;
+}
+
 int blocks_for(int ntiles, int lanes_per_block) {
   int dev = 0, cus = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
@@ -613,7 +666,7 @@ static bool region_plan(const agd_eikonal_desc* d, const int* box, int waves, si
 // One solve of this kind at a time on a device: its workgroups wait for each
 // other, so two of them could each hold half of the compute units.  A solve
 // that finds another one running takes the pass solver instead.
-static std::mutex g_region_mutex[64];
+static std::mutex g_region_mutex[kMaxDevices];
 
 template <class S> static RegionKernels<S> region_lookup(int model, int d) {
   switch (model) {
@@ -636,7 +689,7 @@ static int region_impl(Workspace& ws, const EikArgs<S>& e, const agd_eikonal_des
   RegionPlan p;
   int dev = 0;
   const RegionKernels<S> rk = region_lookup<S>(d->model, d->ndim);
-  if (!rk.solve || hipGetDevice(&dev) != hipSuccess || dev >= 64 || !region_plan(d, rk.box, rk.waves, rk.lds, p))
+  if (!rk.solve || hipGetDevice(&dev) != hipSuccess || dev >= kMaxDevices || !region_plan(d, rk.box, rk.waves, rk.lds, p))
     return AGD_OK;
   std::unique_lock<std::mutex> lock(g_region_mutex[dev], std::try_to_lock);
   if (!lock.owns_lock()) return AGD_OK;
@@ -683,6 +736,7 @@ static int region_impl(Workspace& ws, const EikArgs<S>& e, const agd_eikonal_des
   const size_t lds = rk.lds(p.ntot);
   AGD_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(rk.solve),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
+  ws.busy = true;
   AGD_HIP_TRY(hipEventRecord(ws.ev0, stream));
   fill_i32(reinterpret_cast<int32_t*>(base), int64_t(b_zero / 4), 0, stream);
   const unsigned wg = unsigned(ceil_div(ntiles, 4));
@@ -694,6 +748,7 @@ static int region_impl(Workspace& ws, const EikArgs<S>& e, const agd_eikonal_des
   touched = true;
   AGD_HIP_TRY(hipMemcpyAsync(ws.host_counts, a.ctl, kRegionCtl * 4, hipMemcpyDeviceToHost, stream));
   AGD_HIP_TRY(hipStreamSynchronize(stream));
+  ws.busy = false;
   const uint32_t* c = reinterpret_cast<const uint32_t*>(ws.host_counts);
   if (c[kRegionFinished] != 1u) return AGD_OK;
   taken = true;
@@ -752,7 +807,6 @@ static int solve_impl(Workspace& ws, const agd_eikonal_desc* d, const agd_eikona
   // Fields of 4 GiB or more go to the general variant (64-bit addressing).
   const bool big = uint64_t(g.size_tot) * sizeof(S) > uint64_t(0xffffffffu);
   AGD_REQUIRE(!pre || !big, "a precomputed scheme needs fields below 4 GiB (2^30 FP32 cells)");
-  // Zeroed bytes, padding included: the argument bytes key the graph cache.
   EikArgs<S> a;
   std::memset(&a, 0, sizeof a);
   a.u = static_cast<S*>(io->values);
@@ -841,23 +895,16 @@ static int solve_impl(Workspace& ws, const agd_eikonal_desc* d, const agd_eikona
                            : ((io->wall_dist || g.periodic || factor || big || bab)
                                   ? ks.update_walls
                                   : ks.update);
-  auto launch = [&](int32_t koff, hipStream_t s, bool phase) {
+  auto launch = [&](int32_t koff, hipStream_t s) {
     a.w.koff = koff;
-    a.w.phase_from_koff = phase ? 1 : 0;
     hipLaunchKernelGGL(kern, dim3(blocks), dim3(ni), 0, s, a);
     if (bab)
       hipLaunchKernelGGL(bab_threshold_kernel, dim3(1), dim3(64), 0, s, a.bab.ctl,
                          int64_t(d->bound_active_blocks), d->minchg_delta_min);
   };
-  auto key = [&](std::vector<unsigned char>& k) {
-    key_append(k, kern);
-    key_append(k, a);
-    key_append(k, d->bound_active_blocks);
-    key_append(k, d->minchg_delta_min);
-  };
   WorklistResult r;
   int st = run_worklist(ws, g.ntiles, blocks, d->nitermax_o, d->check_interval, stream, init, launch,
-                        key, r, d->time_launches != 0, d->use_graph != 0);
+                        r, d->time_launches != 0, d->use_graph != 0);
   if (st) return st;
   if (stats) {
     stats->kernel_ms = r.kernel_ms;
@@ -1041,18 +1088,13 @@ static int solve_batched_impl(Workspace& ws, const agd_eikonal_desc* d, int32_t 
     }
     return AGD_OK;
   };
-  auto launch = [&](int32_t koff, hipStream_t s, bool phase) {
+  auto launch = [&](int32_t koff, hipStream_t s) {
     a.w.koff = koff;
-    a.w.phase_from_koff = phase ? 1 : 0;
     hipLaunchKernelGGL(ks.update_batch, dim3(blocks), dim3(ks.block), 0, s, a);
-  };
-  auto key = [&](std::vector<unsigned char>& k) {
-    key_append(k, ks.update_batch);
-    key_append(k, a);
   };
   WorklistResult r;
   st = run_worklist(ws, int32_t(tiles), blocks, d->nitermax_o, d->check_interval, stream, init,
-                    launch, key, r, d->time_launches != 0, d->use_graph != 0, kb);
+                    launch, r, d->time_launches != 0, d->use_graph != 0, kb);
   if (st) return st;
   if (stats) {
     stats->kernel_ms = r.kernel_ms;
@@ -1107,7 +1149,7 @@ using namespace agd;
 struct agd_solver {
   int device = 0;
   hipStream_t stream = nullptr;
-  Workspace ws;
+  WorkspaceLease ws;
 };
 
 namespace agd {
@@ -1165,7 +1207,6 @@ static int check_entry(int32_t* cnt, const agd_eikonal_desc* desc, const agd_eik
 constexpr size_t kScratchBytes = size_t(12) << 20;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
-constexpr int kMaxDevices = 64;
 static std::once_flag g_scratch_once[kMaxDevices];
 static void* g_scratch_addr[kMaxDevices];
 static hipError_t g_scratch_err[kMaxDevices];
@@ -1265,7 +1306,7 @@ int agd_solver_create(const agd_eikonal_desc* desc, void* stream, agd_solver** o
     const GridDesc g = make_grid(desc);
     int ni = 1;
     for (int k = 0; k < desc->ndim; ++k) ni *= desc->shape_i[k];
-    const int st = s->ws.ensure(g.ntiles, shard_capacity(g.ntiles, blocks_for(g.ntiles, ni)),
+    const int st = s->ws->ensure(g.ntiles, shard_capacity(g.ntiles, blocks_for(g.ntiles, ni)),
                                 hist_len(desc->nitermax_o, desc->check_interval));
     if (st) {
       delete s;
@@ -1273,6 +1314,25 @@ int agd_solver_create(const agd_eikonal_desc* desc, void* stream, agd_solver** o
     }
   }
   *out = s;
+  return AGD_OK;
+}
+
+int agd_release_workspaces(int64_t* bytes) {
+  int dev = 0;
+  AGD_HIP_TRY(hipGetDevice(&dev));
+  AGD_REQUIRE(dev >= 0 && dev < kMaxDevices, "device index beyond the workspace table");
+  std::vector<Workspace*> idle;
+  {
+    WorkspacePool& p = pool_of(dev);
+    std::lock_guard<std::mutex> lock(p.mutex);
+    idle.swap(p.idle);
+  }
+  int64_t n = 0;
+  for (Workspace* w : idle) {
+    n += int64_t(w->bytes());
+    delete w;
+  }
+  if (bytes) *bytes = n;
   return AGD_OK;
 }
 
@@ -1290,7 +1350,7 @@ int agd_solver_solve(agd_solver* s, const agd_eikonal_desc* desc, const agd_eiko
                      agd_eikonal_stats* stats) {
   const int st = check_handle(s);
   if (st) return st;
-  return solve_entry(s->ws, desc, io, stats, s->stream);
+  return solve_entry(*s->ws, desc, io, stats, s->stream);
 }
 
 int agd_solver_solve_batched(agd_solver* s, const agd_eikonal_desc* desc, int32_t ninst,
@@ -1298,25 +1358,25 @@ int agd_solver_solve_batched(agd_solver* s, const agd_eikonal_desc* desc, int32_
                              agd_eikonal_stats* stats) {
   const int st = check_handle(s);
   if (st) return st;
-  return batched_entry(s->ws, desc, ninst, instances, io, stats, s->stream);
+  return batched_entry(*s->ws, desc, ninst, instances, io, stats, s->stream);
 }
 
 int agd_solver_check(agd_solver* s, const agd_eikonal_desc* desc, const agd_eikonal_io* io,
                      double atol, double rtol, int64_t* violations) {
   int st = check_handle(s);
   if (st) return st;
-  st = s->ws.ensure(1, 1, 1);
+  st = s->ws->ensure(1, 1, 1);
   if (st) return st;
-  return check_entry(s->ws.check_count, desc, io, atol, rtol, violations, s->stream);
+  return check_entry(s->ws->check_count, desc, io, atol, rtol, violations, s->stream);
 }
 
 int agd_solver_check_stale(agd_solver* s, const agd_eikonal_desc* desc, const agd_eikonal_io* io,
                            double atol, double rtol, uint32_t* stale_bits, int64_t* stale) {
   int st = check_handle(s);
   if (st) return st;
-  st = s->ws.ensure(1, 1, 1);
+  st = s->ws->ensure(1, 1, 1);
   if (st) return st;
-  return check_entry(s->ws.check_count, desc, io, atol, rtol, stale, s->stream, true, stale_bits);
+  return check_entry(s->ws->check_count, desc, io, atol, rtol, stale, s->stream, true, stale_bits);
 }
 
 int agd_solver_repair(agd_solver* s, const agd_eikonal_desc* desc, const agd_eikonal_io* io,
@@ -1324,17 +1384,17 @@ int agd_solver_repair(agd_solver* s, const agd_eikonal_desc* desc, const agd_eik
                       int32_t* rounds) {
   int st = check_handle(s);
   if (st) return st;
-  st = s->ws.ensure(1, 1, 1);
+  st = s->ws->ensure(1, 1, 1);
   if (st) return st;
-  return repair_entry(s->ws.check_count, desc, io, atol, rtol, max_rounds, violations_left, rounds,
+  return repair_entry(s->ws->check_count, desc, io, atol, rtol, max_rounds, violations_left, rounds,
                       s->stream);
 }
 
 int agd_eikonal_solve_batched(const agd_eikonal_desc* desc, int32_t ninst,
                               const agd_batch_instance* instances, const agd_eikonal_io* io,
                               agd_eikonal_stats* stats, void* stream) {
-  Workspace ws;  // this call's own, released on return
-  return batched_entry(ws, desc, ninst, instances, io, stats, as_stream(stream));
+  WorkspaceLease ws;  // this call's own
+  return batched_entry(*ws, desc, ninst, instances, io, stats, as_stream(stream));
 }
 
 int agd_scheme_supported(int32_t model, int32_t ndim, const int32_t* shape_i) {
@@ -1370,8 +1430,8 @@ int agd_batch_tile_supported(int32_t model, int32_t ndim, const int32_t* shape_i
 
 int agd_eikonal_solve(const agd_eikonal_desc* desc, const agd_eikonal_io* io,
                       agd_eikonal_stats* stats, void* stream) {
-  Workspace ws;  // this call's own, released on return
-  return solve_entry(ws, desc, io, stats, as_stream(stream));
+  WorkspaceLease ws;  // this call's own
+  return solve_entry(*ws, desc, io, stats, as_stream(stream));
 }
 
 int agd_geodesic_ode_online(const agd_eikonal_desc* desc, const agd_eikonal_io* io,

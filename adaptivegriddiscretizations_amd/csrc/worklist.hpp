@@ -5,15 +5,17 @@
 // activates to list[(k+1)%2] / count[(k+1)%3] (deduplicated by a per-tile
 // stamp: atomicMax(stamp, k+1) returns a smaller value exactly once per pass)
 // and zeroes count[(k+2)%3], the counter of pass k+1's successor.  No pass
-// ever clears a list or a flag array, so a solve costs one launch per pass
-// plus one 4-byte read-back every `check_interval` passes.  This replaces
-// the reference's per-pass host round trip (np.any + flatnonzero + fill,
-// _solvers.py:184-190, _StopCriterion.py:62-82).
+// ever clears a list or a flag array, so a solve costs one launch per pass;
+// each pass writes its list length to host memory, where the host, some passes
+// ahead, sees the first empty one.  This replaces the reference's per-pass host
+// round trip (np.any + flatnonzero + fill, _solvers.py:184-190,
+// _StopCriterion.py:62-82).
 #pragma once
 
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <chrono>
 #include <vector>
 
 #include "common.hpp"
@@ -28,8 +30,7 @@ constexpr int kShards = 64;
 constexpr int kCountStride = 16;                         // one 64-byte line per counter
 constexpr int kRow = kShards * kCountStride;             // one pass's counters
 constexpr int kFixedIdx = 3 * kRow;                      // fixed-list length (global iteration)
-constexpr int kBaseIdx = 3 * kRow + kCountStride;        // pass base
-constexpr int kCountsLen = 3 * kRow + 2 * kCountStride;  // cleared at the start of a solve
+constexpr int kCountsLen = 3 * kRow + kCountStride;      // cleared at the start of a solve
 constexpr int kSumIdx = kCountsLen;                      // int64[2]: non-empty passes, visits
 constexpr int kCountsAlloc = kCountsLen + 4;
 
@@ -55,7 +56,9 @@ struct Workspace {
   int32_t* bab = nullptr;     // bound_active_blocks control block (kBabLen)
   int32_t* lists = nullptr;   // 2 * kShards * shard_cap
   int32_t* counts = nullptr;  // kCountsLen
-  int32_t* hist = nullptr;    // hist_cap: list length of every pass
+  // hist_cap: list length of every pass; pinned host memory that the kernels
+  // write to (fixed region: device memory)
+  int32_t* hist = nullptr;
   int32_t* score = nullptr;   // 2 * tile_cap (FIM scores; fixed list of global iteration)
   int32_t* check_count = nullptr;  // residual-check counter
   void* inst = nullptr;            // batched solves: instance table (inst_cap InstDesc)
@@ -65,21 +68,14 @@ struct Workspace {
   void* region = nullptr;          // one-launch solve: control words, tile blocks (region_bytes)
   size_t region_bytes = 0;
   int64_t tile_cap = 0, shard_cap = 0, hist_cap = 0, inst_cap = 0, tinst_cap = 0;
-  // Host side.  host_counts: pinned (owned) or host_local (fixed region),
-  // 2 * kRow entries, two chunks in flight.
+  void* scratch = nullptr;         // linear systems: rows (scratch_bytes)
+  size_t scratch_bytes = 0;
+  // Host side.  host_counts: pinned (owned) or host_local (fixed region), kRow entries.
   int32_t* host_counts = nullptr;
-  int32_t host_local[2 * kRow];
+  int32_t host_local[kRow];
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
-  hipEvent_t chunk_ev[2] = {nullptr, nullptr};  // list length of a chunk copied
-  // Private stream used only to record pass chunks into a graph (the legacy
-  // null stream, torch's default, cannot be captured).  Nothing executes on
-  // it: the instantiated graph is launched on the caller's stream.
-  hipStream_t capture_stream = nullptr;
-  // Last instantiated pass chunk and the bytes (kernel, arguments, grid,
-  // chunk length) it was captured with: a solve with identical bytes
-  // replays it instead of capturing again.
-  hipGraphExec_t exec = nullptr;
-  std::vector<unsigned char> exec_key;
+  // Work that uses the buffers may still be queued (a call that failed half way).
+  bool busy = false;
   // Fixed region (allocation-free entry point): nothing is ever allocated,
   // grown or freed, no events are recorded and passes launch eagerly.
   bool fixed = false;
@@ -98,6 +94,10 @@ struct Workspace {
   int ensure_ftab(size_t bytes);
   // One-launch solve: a buffer of at least `bytes`.
   int ensure_region(size_t bytes);
+  // Linear systems: a buffer of at least `bytes`.
+  int ensure_scratch(size_t bytes);
+  // Device bytes held.
+  size_t bytes() const;
   // Frees everything owned (no-op for a fixed region).
   void release();
   // Lays the buffers out in [base, base + bytes) (fixed region); AGD_EINVAL
@@ -105,6 +105,27 @@ struct Workspace {
   int bind_fixed(void* base, size_t bytes, int64_t ntiles, int64_t shard_cap, int64_t nhist);
   // Bytes bind_fixed needs.
   static size_t fixed_bytes(int64_t ntiles, int64_t shard_cap, int64_t nhist);
+};
+
+// A workspace of the current device, taken from the idle ones when there is
+// one (an allocation costs 20 to 400 us and a free waits for the device; a call
+// of the Python driver makes and drops a handle).  Given back on destruction
+// once its work has completed; at most kPoolMost idle ones of kPoolBytes in
+// all are kept per device, and agd_release_workspaces frees them.
+constexpr size_t kPoolMost = 4;
+constexpr size_t kPoolBytes = size_t(2) << 30;
+class WorkspaceLease {
+ public:
+  WorkspaceLease();
+  ~WorkspaceLease();
+  WorkspaceLease(const WorkspaceLease&) = delete;
+  WorkspaceLease& operator=(const WorkspaceLease&) = delete;
+  Workspace& operator*() { return *ws_; }
+  Workspace* operator->() { return ws_; }
+
+ private:
+  int device_ = -1;
+  Workspace* ws_;
 };
 
 // Workgroups of a pass launch: enough resident waves per CU of the current
@@ -120,12 +141,6 @@ __global__ inline void fill_i32_kernel(int32_t* p, int64_t n, int32_t v) {
 inline void fill_i32(int32_t* p, int64_t n, int32_t v, hipStream_t s) {
   if (n <= 0) return;
   hipLaunchKernelGGL(fill_i32_kernel, dim3(unsigned((n + 255) / 256)), dim3(256), 0, s, p, n, v);
-}
-
-// Appends the bytes of `x` to a graph cache key.
-template <class T> inline void key_append(std::vector<unsigned char>& k, const T& x) {
-  const unsigned char* p = reinterpret_cast<const unsigned char*>(&x);
-  k.insert(k.end(), p, p + sizeof(T));
 }
 
 // Capacity of one sub-list.  A pass appends at most 2d+1 <= 7 tiles per
@@ -171,10 +186,8 @@ __device__ inline void enqueue_wave(bool want, int32_t tile, int32_t entry, int3
 }
 
 // Worklist state seen by a pass kernel.  counts holds three rows of kShards
-// rotating sub-list lengths, the fixed-list length and the pass base.  A
-// kernel runs pass iter = counts[kBaseIdx] + koff, so a chunk of passes with
-// koff = 0..G-1 followed by an advance of the base by G can be captured once
-// as a graph and replayed.
+// rotating sub-list lengths and the fixed-list length; koff is the number of
+// the pass, so a wave loads only its row.
 struct WorkCtx {
   int32_t* lists;          // 2 * kShards * shard_cap entries
   int32_t* counts;         // kCountsLen
@@ -185,10 +198,6 @@ struct WorkCtx {
   int32_t tile_cap;
   int32_t shard_cap;
   int32_t koff;
-  // 1 when the pass number is koff modulo 6 (eager passes: base 0; graph
-  // chunks of a multiple of 6 passes): the counter row and the list parity
-  // then follow from koff, and a wave loads only its row.
-  int32_t phase_from_koff;
 };
 
 struct PassView {
@@ -203,28 +212,16 @@ struct PassView {
   int32_t* score_next;
 };
 
-// Every wave loads the three counter rows and the pass base at once (no
-// dependent load), keeps its pass's row as a prefix sum across lanes (lane
-// s = sub-list s).  Block 0 zeroes the row of pass iter+2 and records the
-// list length.  Must be called by every thread of the block.
+// Every wave loads its pass's row and keeps it as a prefix sum across lanes
+// (lane s = sub-list s).  Block 0 zeroes the row of pass iter+2 and records
+// the list length.  Must be called by every thread of the block.
 __device__ inline PassView pass_begin(const WorkCtx& c) {
   const int lane = threadIdx.x & 63;
-  const int base = c.counts[kBaseIdx];
   const int fixed_n = c.counts[kFixedIdx];
   PassView v;
-  v.iter = base + c.koff;
-  int mine, par;
-  if (c.phase_from_koff) {
-    mine = c.counts[(c.koff % 3) * kRow + lane * kCountStride];
-    par = c.koff & 1;
-  } else {
-    const int c0 = c.counts[0 * kRow + lane * kCountStride];
-    const int c1 = c.counts[1 * kRow + lane * kCountStride];
-    const int c2 = c.counts[2 * kRow + lane * kCountStride];
-    const int r = v.iter % 3;
-    mine = r == 0 ? c0 : (r == 1 ? c1 : c2);
-    par = v.iter & 1;
-  }
+  v.iter = c.koff;
+  const int mine = c.counts[(c.koff % 3) * kRow + lane * kCountStride];
+  const int par = c.koff & 1;
   int incl = mine;
 #pragma unroll
   for (int d = 1; d < 64; d <<= 1) {
@@ -244,7 +241,8 @@ __device__ inline PassView pass_begin(const WorkCtx& c) {
   v.score_next = c.score + (v.iter & 1) * c.tile_cap;
   if (blockIdx.x == 0 && threadIdx.x < 64) {
     c.counts[((v.iter + 2) % 3) * kRow + lane * kCountStride] = 0;
-    if (lane == 0) c.hist[v.iter] = v.count;
+    // (read by the host while later passes run)
+    if (lane == 0) __hip_atomic_store(c.hist + v.iter, v.count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   }
   return v;
 }
@@ -257,8 +255,6 @@ __device__ inline int32_t pass_entry(const PassView& v, int li) {
   const int excl = s == 0 ? 0 : __shfl(v.incl, s - 1);
   return v.list_in[int64_t(s) * v.shard_cap + (li - excl)];
 }
-
-__global__ inline void advance_kernel(int32_t* counts, int32_t g) { counts[kBaseIdx] += g; }
 
 // out[0] = passes with a non-empty list, out[1] = tile visits, over hist[0..n).
 // One workgroup of 256 lanes.
@@ -368,34 +364,40 @@ inline int64_t hist_len(int64_t nitermax, int check_interval) {
   return nitermax + std::max(1, check_interval) + 8;
 }
 
+// Passes queued beyond the last one that the host has seen begin.  A launch
+// costs the host about 3 us and a pass takes 8 us or more, so a few would
+// do; the rest covers the host being kept away.  Each one too many at the end
+// is an empty pass of 2 us.
+constexpr int kAhead = 10;
+
 // Runs passes until the list empties or nitermax passes were issued.
 // `init(ws)` enqueues the initial list into the sub-lists of pass 0 (list
-// row 0, counter row 0); `launch(koff, stream)` enqueues one pass of
-// iteration base + koff on `stream`, on a grid of `grid` workgroups.
-// With `graph`, chunks of `check_interval` passes are captured into a
-// hipGraph and replayed; `key(k)` appends to k the bytes the captured
-// launches depend on (kernel, arguments, grid), and the workspace's last
-// graph is replayed when they are unchanged.  The host reads the next list
-// length after each chunk.  Optional per-pass timing records an event pair
-// around every pass (and then launches eagerly).  A fixed-region workspace
-// launches eagerly and records no event.
-template <class Init, class Launch, class Key>
+// row 0, counter row 0); `launch(k, stream)` enqueues pass k on `stream`, on a
+// grid of `grid` workgroups.  With `ahead` (and no per-pass timing), the host
+// queues passes as long as fewer than kAhead of them have not begun, and stops
+// when one begins with an empty list: its length in pinned memory is all that
+// the host waits for.  (Chunks of passes captured in a graph need a capture
+// whenever an argument changes and the length copied back after each: whole
+// calls of riemann2 2000^2, rander2 501 x 403 and riemann3 200^3 took 5.25, 4.05 and
+// 5.68 ms with them, 5.0, 3.7 and 5.55 ms launched one by one with the same checks.)  Without, the
+// host reads the next list length every `check_interval` passes; per-pass
+// timing records an event pair around every pass.
+template <class Init, class Launch>
 int run_worklist(Workspace& wsr, int32_t ntiles, int32_t grid, int64_t nitermax, int check_interval,
-                 hipStream_t stream, Init init, Launch launch, Key key, WorklistResult& res,
-                 bool time_launches = false, bool graph = false, int tiles_per_block = 1) {
+                 hipStream_t stream, Init init, Launch launch, WorklistResult& res,
+                 bool time_launches = false, bool ahead = false, int tiles_per_block = 1) {
   Workspace* ws = &wsr;
   const int ci = std::max(1, check_interval);
   const int64_t nhist = hist_len(nitermax, ci);
   int st = ws->ensure(ntiles, shard_capacity(ntiles, grid, tiles_per_block), nhist);
   if (st) return st;
-  if (ws->fixed) {
-    time_launches = false;
-    graph = false;
-  }
+  if (ws->fixed) time_launches = ahead = false;
+  ahead = ahead && !time_launches;
   int32_t* counts = ws->counts;
+  ws->busy = true;
   fill_i32(ws->stamp, ntiles, -1, stream);
   fill_i32(counts, kCountsLen, 0, stream);
-  fill_i32(ws->hist, nhist, 0, stream);
+  if (ws->fixed) fill_i32(ws->hist, nhist, 0, stream);
   st = init(ws);
   if (st) return st;
   AGD_HIP_TRY(hipGetLastError());
@@ -425,44 +427,6 @@ int run_worklist(Workspace& wsr, int32_t ntiles, int32_t grid, int64_t nitermax,
     return AGD_OK;
   };
 
-  // Per-launch timing needs event pairs around every launch, which a graph
-  // does not record: timed runs launch eagerly.
-  graph = graph && !time_launches;
-  hipGraphExec_t exec = nullptr;
-  if (graph) {
-    std::vector<unsigned char> k;
-    key(k);
-    key_append(k, grid);
-    key_append(k, ci);
-    if (ws->exec && k == ws->exec_key) {
-      exec = ws->exec;
-    } else {
-      if (ws->exec) {
-        (void)hipGraphExecDestroy(ws->exec);
-        ws->exec = nullptr;
-        ws->exec_key.clear();
-      }
-      hipGraph_t g = nullptr;
-      hipStream_t cs = ws->capture_stream;
-      AGD_HIP_TRY(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
-      for (int i = 0; i < ci; ++i) launch(i, cs, ci % 6 == 0);
-      hipLaunchKernelGGL(advance_kernel, dim3(1), dim3(1), 0, cs, counts, ci);
-      // End the capture whatever happened inside it, so the stream is usable again.
-      const hipError_t cap_err = hipGetLastError();
-      const hipError_t end_err = hipStreamEndCapture(cs, &g);
-      if (cap_err != hipSuccess || end_err != hipSuccess) {
-        if (g) (void)hipGraphDestroy(g);
-        AGD_HIP_TRY(cap_err);
-        AGD_HIP_TRY(end_err);
-      }
-      const hipError_t inst_err = hipGraphInstantiate(&exec, g, nullptr, nullptr, 0);
-      (void)hipGraphDestroy(g);
-      AGD_HIP_TRY(inst_err);
-      ws->exec = exec;
-      ws->exec_key = std::move(k);
-    }
-  }
-
   const bool timed = ws->ev0 != nullptr;
   if (timed) AGD_HIP_TRY(hipEventRecord(ws->ev0, stream));
   int64_t k = 0;
@@ -472,38 +436,51 @@ int run_worklist(Workspace& wsr, int32_t ntiles, int32_t grid, int64_t nitermax,
     for (int sh = 0; sh < kShards; ++sh) n += row[sh * kCountStride];
     return n;
   };
-  if (graph) {
-    // Pipelined chunks: chunk c+1 is queued before the host looks at the
-    // list length left by chunk c (copied right behind chunk c, ahead of
-    // chunk c+1 in stream order), so the device never idles on the host's
-    // check.  The chunk queued after convergence runs empty passes.
-    int slot = 0;
-    AGD_HIP_TRY(hipGraphLaunch(exec, stream));
-    k += ci;
-    AGD_HIP_TRY(hipMemcpyAsync(ws->host_counts, counts + (k % 3) * kRow, kRow * sizeof(int32_t),
-                               hipMemcpyDeviceToHost, stream));
-    AGD_HIP_TRY(hipEventRecord(ws->chunk_ev[0], stream));
-    while (true) {
-      const bool more = k < nitermax;
-      if (more) {
-        AGD_HIP_TRY(hipGraphLaunch(exec, stream));
-        k += ci;
-        AGD_HIP_TRY(hipMemcpyAsync(ws->host_counts + (1 - slot) * kRow, counts + (k % 3) * kRow,
-                                   kRow * sizeof(int32_t), hipMemcpyDeviceToHost, stream));
-        AGD_HIP_TRY(hipEventRecord(ws->chunk_ev[1 - slot], stream));
+  if (ahead) {
+    volatile int32_t* const len = ws->hist;
+    int64_t begun = 0;  // passes known to have begun
+    int idle = 0;
+    auto last_look = std::chrono::steady_clock::now();
+    while (!converged && begun < nitermax) {
+      if (k < nitermax && k - begun < kAhead) {
+        len[k] = -1;
+        launch(int32_t(k), stream);
+        AGD_HIP_TRY(hipGetLastError());
+        ++k;
+        idle = 0;
       }
-      AGD_HIP_TRY(hipEventSynchronize(ws->chunk_ev[slot]));
-      if (list_length(ws->host_counts + slot * kRow) == 0) {
-        converged = true;
-        break;
+      if (len[begun] >= 0) {
+        converged = len[begun] == 0;
+        ++begun;
+        idle = 0;
+      } else if (++idle > 4096) {
+        // nothing for a while: let a failure of the stream end the wait
+        idle = 0;
+        const auto now = std::chrono::steady_clock::now();
+        if (now - last_look > std::chrono::milliseconds(20)) {
+          last_look = now;
+          const hipError_t e = hipStreamQuery(stream);
+          if (e != hipErrorNotReady) {
+            AGD_HIP_TRY(e);
+            if (len[begun] < 0) {
+              set_error("a pass of the worklist did not run");
+              return AGD_EHIP;
+            }
+          }
+        }
       }
-      if (!more) break;
-      slot = 1 - slot;
+    }
+    AGD_HIP_TRY(hipGetLastError());
+    if (!converged) {
+      AGD_HIP_TRY(hipMemcpyAsync(ws->host_counts, counts + (k % 3) * kRow, kRow * sizeof(int32_t),
+                                 hipMemcpyDeviceToHost, stream));
+      AGD_HIP_TRY(hipStreamSynchronize(stream));
+      converged = list_length(ws->host_counts) == 0;
     }
   } else {
     while (k < nitermax) {
       if (time_launches) AGD_HIP_TRY(hipEventRecord(evs[2 * pending], stream));
-      launch(int32_t(k), stream, true);
+      launch(int32_t(k), stream);
       if (time_launches) AGD_HIP_TRY(hipEventRecord(evs[2 * pending + 1], stream));
       ++pending;
       ++k;
@@ -535,13 +512,22 @@ int run_worklist(Workspace& wsr, int32_t ntiles, int32_t grid, int64_t nitermax,
     const int st2 = drain();
     if (st2) return st2;
   }
-  // Non-empty passes and visits, summed on the device from the histogram.
-  int64_t* sums = reinterpret_cast<int64_t*>(counts + kSumIdx);
-  hipLaunchKernelGGL(hist_sum_kernel, dim3(1), dim3(256), 0, stream, ws->hist, k, sums);
-  AGD_HIP_TRY(hipGetLastError());
+  // Non-empty passes and visits.
   int64_t hs[2] = {0, 0};
-  AGD_HIP_TRY(hipMemcpyAsync(hs, sums, sizeof(hs), hipMemcpyDeviceToHost, stream));
-  AGD_HIP_TRY(hipStreamSynchronize(stream));
+  if (ws->fixed) {
+    int64_t* sums = reinterpret_cast<int64_t*>(counts + kSumIdx);
+    hipLaunchKernelGGL(hist_sum_kernel, dim3(1), dim3(256), 0, stream, ws->hist, k, sums);
+    AGD_HIP_TRY(hipGetLastError());
+    AGD_HIP_TRY(hipMemcpyAsync(hs, sums, sizeof(hs), hipMemcpyDeviceToHost, stream));
+    AGD_HIP_TRY(hipStreamSynchronize(stream));
+  } else {
+    AGD_HIP_TRY(hipStreamSynchronize(stream));
+    for (int64_t i = 0; i < k; ++i) {
+      hs[0] += ws->hist[i] > 0 ? 1 : 0;
+      hs[1] += ws->hist[i];
+    }
+  }
+  ws->busy = false;
   res.passes = k;
   res.niter = hs[0];
   res.visits = hs[1];

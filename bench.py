@@ -194,7 +194,7 @@ def main():
                     help='store the stencils once per solve (precompute_scheme) instead of rebuilding '
                          'them in registers at every tile visit')
     ap.add_argument('--no-graph', action='store_true',
-                    help='launch every pass eagerly instead of replaying captured pass chunks')
+                    help='wait for the list length every check_interval passes instead of queueing passes ahead')
     ap.add_argument('--copy-calibration', type=int, default=0, metavar='MIB',
                     help='only run a plain device copy of MIB MiB three times (reference for '
                          'the FETCH_SIZE / WRITE_SIZE counters) and exit')
@@ -304,7 +304,7 @@ def main():
             "model": wl.model, "grid": list(wl.dims), "tile": list(iface.shape_i),
             "niter_i": iface.niter_i, "solver": iface.solver, "atol": iface.atol, "rtol": iface.rtol,
             "parallelism": "single GPU",
-            "pass_launch": "eager" if args.no_graph else "hipGraph",
+            "pass_launch": "checked every check_interval" if args.no_graph else "queued ahead",
             "precompute_scheme": bool(iface.precompute_scheme),
         },
         "solved_cells_per_s": wl.ncells * args.steps / wall,

@@ -80,12 +80,11 @@ typedef struct agd_eikonal_desc {
   double atol, rtol;      /* |u_old-u_new| <= atol + rtol |u_new|        */
   int64_t nitermax_o;     /* maximum number of grid-level passes         */
   double iso_weights[3];  /* AGD_ISOTROPIC: per-axis weights (h^-2)      */
-  int32_t check_interval; /* passes between host convergence checks (>=1);
-                             with use_graph, a multiple of 6 lets every pass
-                             read only its own row of worklist counters */
+  int32_t check_interval; /* without use_graph: passes between host convergence checks (>=1) */
   int32_t activate_all;   /* 1: start with every tile active (warm start) */
   int32_t time_launches;  /* 1: time every pass with an event pair (kernel_ms) */
-  int32_t use_graph;      /* 1: capture check_interval passes once as a hipGraph and replay it */
+  int32_t use_graph;      /* 1: the host queues passes ahead of the device and sees each begin;
+                             0: it waits for the list length every check_interval passes */
   int32_t order;          /* 1 (or 0) or 2: second-order upwind differences
                              where the solution is smooth (HFM.h:91-134) */
   int32_t convex;         /* curvature models ReedsSheppForward2, Elastica2,
@@ -201,6 +200,10 @@ int agd_device_count(int32_t* count);
 typedef struct agd_solver agd_solver;
 int agd_solver_create(const agd_eikonal_desc* desc, void* stream, agd_solver** out);
 int agd_solver_destroy(agd_solver* solver);
+/* A workspace whose owner is gone and whose work has completed is kept for the
+ * next handle or call (per device: at most 4, 2 GiB in all).  Frees those of the
+ * current device; *bytes (nullable) receives their size. */
+int agd_release_workspaces(int64_t* bytes);
 /* agd_eikonal_solve, agd_eikonal_solve_batched and agd_eikonal_check through
  * a handle, on its stream. */
 int agd_solver_solve(agd_solver* solver, const agd_eikonal_desc* desc, const agd_eikonal_io* io,
