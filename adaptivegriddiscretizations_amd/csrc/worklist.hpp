@@ -379,7 +379,7 @@ constexpr int kAhead = 10;
 // the host waits for.  (Chunks of passes captured in a graph need a capture
 // whenever an argument changes and the length copied back after each: whole
 // calls of riemann2 2000^2, rander2 501 x 403 and riemann3 200^3 took 5.25, 4.05 and
-// 5.68 ms with them, 5.0, 3.7 and 5.55 ms launched one by one with the same checks.)  Without, the
+// 5.68 ms with them, 4.65, 3.15 and 4.99 ms with passes queued ahead.)  Without, the
 // host reads the next list length every `check_interval` passes; per-pass
 // timing records an event pair around every pass.
 template <class Init, class Launch>
