@@ -42,6 +42,7 @@ __device__ inline float sqrt_fast(float a) { return __builtin_amdgcn_sqrtf(a); }
 __device__ inline double sqrt_fast(double a) { return __builtin_sqrt(a); }
 __device__ inline float div_fast(float a, float b) { return a * __builtin_amdgcn_rcpf(b); }
 __device__ inline double div_fast(double a, double b) { return a / b; }
+__device__ inline void compiler_fence() { asm volatile("" ::: "memory"); }
 __device__ inline bool isnan_(float a) { return a != a; }
 __device__ inline bool isnan_(double a) { return a != a; }
 
@@ -954,7 +955,10 @@ template <class S, int N> __device__ inline void sort_pairs(S (&v)[N], S (&w)[N]
 
 // HFM.h:165-195: smallest solution of sum_k w_k (u - v_k)_+^2 = rhs^2 over
 // the sorted neighbour values, growing the active set while the quadratic is
-// non-positive at the next value.  Inputs by value (sorted copies).
+// non-positive at the next value.  Inputs by value (sorted copies).  (A value
+// outside the active set enters with weight 0: a wave rarely leaves the set
+// early in all of its cells, and without branches the terms of one step
+// overlap with the test of the next.)
 template <class S, int N>
 __device__ inline S hfm_solve(S (&v)[N], S (&w)[N], S rhs) {
   sort_pairs<S, N>(v, w);
@@ -965,11 +969,12 @@ __device__ inline S hfm_solve(S (&v)[N], S (&w)[N], S rhs) {
   for (int k = 1; k < N; ++k) {
     const S t = v[k] - vmin;
     go = go && !((a * t - S(2) * b) * t + c > S(0));
-    if (go) {
-      a += w[k];
-      b += w[k] * t;
-      c += w[k] * t * t;
-    }
+    const S wk = go ? w[k] : S(0);
+    const S tk = go ? t : S(0);
+    const S wt = wk * tk;
+    a += wk;
+    b += wt;
+    c += wt * tk;
   }
   const S delta = b * b - a * c;
   const S sdelta = sqrt_fast(delta > S(0) ? delta : S(0));

@@ -231,6 +231,24 @@ template <int NI> __device__ inline bool block_any(bool p) {
   }
 }
 
+// The same with one barrier, which also ends the LDS accesses before it: flags
+// alternates between two sets of NI / 64 flags.
+template <int NI> __device__ inline bool tile_any(bool p, uint32_t* flags, int& turn) {
+  if constexpr (NI <= 64) {
+    return __ballot(p) != 0;
+  } else {
+    uint32_t* const f = flags + turn * (NI / 64);
+    turn ^= 1;
+    const bool wave = __ballot(p) != 0;
+    if ((threadIdx.x & 63) == 0) f[threadIdx.x >> 6] = wave;
+    __syncthreads();
+    uint32_t any = 0;
+#pragma unroll
+    for (int w = 0; w < NI / 64; ++w) any |= f[w];
+    return any != 0;
+  }
+}
+
 // Block-wide minimum (the same value in every thread).
 template <int NI, class S> __device__ inline S block_min(S v) {
 #pragma unroll
@@ -374,9 +392,16 @@ __global__ void __launch_bounds__(block_lanes<T0 * T1 * T2>(), MODEL == AGD_ELAS
   constexpr int K = tiles_per_block<NI>();
   static_assert(NI % 64 == 0 || (BATCH && 64 % NI == 0),
                 "tiles are whole waves, or (batched solves) pack whole into one wave");
-  // tile g's values at [g * (NI + 1), g * (NI + 1) + NI); slot NI holds 0:
-  // the read of neighbours outside the tile
-  __shared__ S u_s[K * (NI + 1)];
+  // Values outside the tile are read from LDS slots of the lane's own where
+  // no shift is added to them and the tile is one wave: 2 NS registers and
+  // additions fewer.
+  constexpr bool EXT = !GENERAL && !MT::STORED && !MT::DRIFT && NI <= 64;
+  // tile g's values at [g * (NI + 1), g * (NI + 1) + NI), slot NI holding 0;
+  // then with EXT the outside values, for tiles of several waves a second
+  // copy of the values
+  __shared__ S u_s[K * (NI + 1) + (EXT ? NJ * block_lanes<NI>() : (NI > 64 && !MT::STORED ? NI + 1 : 0))];
+  __shared__ uint32_t any_s[NI > 64 ? 2 * (NI / 64) : 1];
+  int turn = 0;
   __shared__ uint8_t wall_s[WALLS ? NI : 1];
 
   const int tid = threadIdx.x;
@@ -480,8 +505,12 @@ __global__ void __launch_bounds__(block_lanes<T0 * T1 * T2>(), MODEL == AGD_ELAS
       if (a.wall) wx = a.wall[n_t];
       wall_s[tid] = uint8_t(wx);
     }
-    us[lt] = seed ? rhs : u_old;
+    S un = seed ? rhs : u_old;
+    us[lt] = un;
     if (lt == 0) us[NI] = S(0);
+    if constexpr (!MT::STORED && NI > 64) {
+      if (lt == 0) u_s[2 * NI + 1] = S(0);
+    }
 
     int code[NJ];
     int code2[ORDER2 ? NJ : 1];
@@ -540,7 +569,6 @@ __global__ void __launch_bounds__(block_lanes<T0 * T1 * T2>(), MODEL == AGD_ELAS
       const int64_t nbox = a.fac.nbox;
       const int64_t fb2 = fb + int64_t(MT::NMIX * NJ) * nbox;  // further neighbours
       __syncthreads();  // u_s complete
-      const bool active = !seed;
       for (int it = 0; it < a.niter_i; ++it) {
         S best = mix_min ? inf_v<S>() : -inf_v<S>();
 #pragma unroll 1
@@ -575,13 +603,13 @@ __global__ void __launch_bounds__(block_lanes<T0 * T1 * T2>(), MODEL == AGD_ELAS
             }
           }
           if constexpr (!MT::CURV)
-            if (a.scode2) order2_correct<S, NS>(us[lt], a.order2_thr, v, v2, w);
+            if (a.scode2) order2_correct<S, NS>(un, a.order2_thr, v, v2, w);
           const S um = hfm_solve<S, NS>(v, w, rhs);
           if (mix_min == (best > um)) best = um;
         }
         __syncthreads();
-        const bool ch = active && (us[lt] > best);
-        if (ch) us[lt] = best;
+        const bool ch = !seed && un > best;
+        if (ch) us[lt] = un = best;
         if (!block_any<NI>(ch)) break;
       }
     } else {
@@ -595,57 +623,101 @@ __global__ void __launch_bounds__(block_lanes<T0 * T1 * T2>(), MODEL == AGD_ELAS
 #pragma unroll
         for (int j = 0; j < NJ; ++j) g2[j] = a.u[code2[j] >= 0 ? code2[j] : n_t];
       }
-      S vo[NJ];
-#pragma unroll
-      for (int j = 0; j < NJ; ++j) vo[j] = code[j] <= -2 ? sh[j] : (code[j] >= 0 ? g[j] + sh[j] : inf_v<S>());
       // LDS slot read at every sweep: the neighbour's own slot inside the
-      // tile, slot NI (holding 0) otherwise, whose value vo then passes
-      // through unchanged (0 + vo == vo up to the sign of a zero, which no
-      // comparison or later sum distinguishes).  The sweep carries no
-      // branch per neighbour.
+      // tile.  Outside: a slot of this lane that holds the gathered value
+      // (EXT), or else slot NI (holding 0), whose value vo then passes through
+      // unchanged (0 + vo == vo up to the sign of a zero, which no comparison
+      // or later sum distinguishes).  The sweep carries no branch per
+      // neighbour.
       int slot[NJ];
+      S vo[EXT ? 1 : NJ];
 #pragma unroll
-      for (int j = 0; j < NJ; ++j) slot[j] = code[j] <= -2 ? -2 - code[j] : NI;
+      for (int j = 0; j < NJ; ++j) {
+        if constexpr (EXT) {
+          const int e = K * (NI + 1) + j * block_lanes<NI>() + tid;
+          u_s[e] = code[j] >= 0 ? g[j] : inf_v<S>();
+          slot[j] = code[j] <= -2 ? grp * (NI + 1) + (-2 - code[j]) : e;
+        } else {
+          vo[j] = code[j] <= -2 ? sh[j] : (code[j] >= 0 ? g[j] + sh[j] : inf_v<S>());
+          slot[j] = code[j] <= -2 ? -2 - code[j] : NI;
+        }
+      }
       __syncthreads();  // u_s complete
 
-      // ---- in-tile sweeps (HFMIter.h:25-84, DECREASING)
-      const bool active = !seed;
-      for (int it = 0; it < a.niter_i; ++it) {
+      // One Jacobi step of the tile, from one copy of its values to another
+      // (or the same: the LDS accesses of one wave are in order).
+      auto sweep = [&](const S* from, S* to) {
+        compiler_fence();
         S v[NS], w[NS];
         S w2v[ORDER2 ? NS : 1];  // further-neighbour values (order 2)
         S x[NJ];
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) x[j] = us[slot[j]];
+        for (int j = 0; j < NJ; ++j) x[j] = EXT ? u_s[slot[j]] : from[slot[j]];
         // Keeps every read unconditional (the compiler would otherwise sink
         // each into a branch with its own wait on the LDS).
 #pragma unroll
         for (int j = 0; j < NJ; ++j) asm volatile("" ::"v"(x[j]));
 #pragma unroll
         for (int k = 0; k < NS; ++k) {
-          const S a0 = x[2 * k] + vo[2 * k];
-          const S a1 = x[2 * k + 1] + vo[2 * k + 1];
+          const S a0 = EXT ? x[2 * k] : x[2 * k] + vo[EXT ? 0 : 2 * k];
+          const S a1 = EXT ? x[2 * k + 1] : x[2 * k + 1] + vo[EXT ? 0 : 2 * k + 1];
           v[k] = (a0 > a1) ? a1 : a0;  // Greater(v,-) keeps the -e side on ties
           w[k] = sw[k];
           if constexpr (ORDER2) {
             // the further neighbour on the chosen side
             const int j2 = 2 * k + ((a0 > a1) ? 1 : 0);
             const int c2 = code2[j2];
-            w2v[k] = c2 <= -2 ? us[-2 - c2] + sh2[j2] : (c2 >= 0 ? g2[j2] + sh2[j2] : inf_v<S>());
+            w2v[k] = c2 <= -2 ? from[-2 - c2] + sh2[j2] : (c2 >= 0 ? g2[j2] + sh2[j2] : inf_v<S>());
           }
         }
-        if constexpr (ORDER2) order2_correct<S, NS>(us[lt], a.order2_thr, v, w2v, w);
-        const S un = hfm_solve<S, NS>(v, w, rhs);
-        __syncthreads();
-        const bool ch = active && (us[lt] > un);
-        if (ch) us[lt] = un;
-        // (packed tiles: the sweeps go on while any tile of the wave
-        // changes; a tile that did not change gives the same values again)
-        if (!block_any<NI>(ch)) break;
+        if constexpr (ORDER2) order2_correct<S, NS>(un, a.order2_thr, v, w2v, w);
+        const S r = hfm_solve<S, NS>(v, w, rhs);
+        un = (!seed && un > r) ? r : un;
+        to[lt] = un;
+        compiler_fence();
+      };
+
+      // ---- in-tile sweeps (HFMIter.h:25-84, DECREASING), until one changes
+      // nothing: the next would read the same values.  Two steps between two
+      // looks, as a step that changes nothing costs less than a look.  (Packed
+      // tiles: the sweeps go on while any tile of the wave changes; a tile
+      // that did not change gives the same values again.)  Tiles of one wave
+      // need no barrier; larger ones alternate between two copies of the
+      // values, one barrier a step.  What bounds a visit is this chain of
+      // dependent steps in 2D (1400 tiles a pass on 1024 SIMDs) and the issue
+      // of vector instructions in 3D (riemann3 200^3: 1600 a visit, 4.6 steps
+      // of 140 in it; about 70 % of the SIMDs' issue slots).  Whole calls, with a
+      // look and two barriers a step and additions for the outside values:
+      // riemann2 2000^2 4.65 ms, here 4.36; riemann3 200^3 5.02, 4.87; 32
+      // images in tiles of 4 waves 4.38, 3.37.
+      if constexpr (NI <= 64) {
+        for (int it = 0; it < a.niter_i;) {
+          const S ub = un;
+          sweep(us, us);
+          if (++it < a.niter_i) {
+            sweep(us, us);
+            ++it;
+          }
+          if (!__any(un < ub)) break;
+        }
+      } else {
+        S* const other = u_s + (NI + 1);
+        for (int it = 0; it < a.niter_i;) {
+          const S ub = un;
+          sweep(us, other);
+          const bool both = ++it < a.niter_i;
+          if (both) {
+            __syncthreads();
+            sweep(other, us);
+            ++it;
+          }
+          const bool more = tile_any<NI>(un < ub, any_s, turn);
+          if (!more || !both) break;
+        }
       }
     }
 
     // ---- store and convergence (Update.h:163-219)
-    const S un = us[lt];
     if (valid) {
       if constexpr (OFF32) st32(a.u, uint32_t(n_t), un);
       else a.u[n_t] = un;
@@ -654,9 +726,8 @@ __global__ void __launch_bounds__(block_lanes<T0 * T1 * T2>(), MODEL == AGD_ELAS
     const S tol = atol + rtol * abs_(un);
     const bool changed = !(isnan_(diff) || diff <= tol);
     if constexpr (K == 1) {
-      any = block_any<NI>(changed);
+      any = tile_any<NI>(changed, any_s, turn);
     } else {
-      __syncthreads();
       const uint64_t m = (uint64_t(1) << NI) - 1;
       any = ((uint64_t(__ballot(changed)) >> (grp * NI)) & m) != 0;
     }

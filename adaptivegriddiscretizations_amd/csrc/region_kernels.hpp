@@ -221,7 +221,6 @@ template <class T> __device__ inline void st_agent(T* p, T v) {
 }
 // Every earlier access of the wave to device memory has completed.
 __device__ inline void wait_memory() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-__device__ inline void compiler_fence() { asm volatile("" ::: "memory"); }
 
 template <int D> __device__ __host__ inline int region_storage(const RegionPlan& p, const int* x) {
   int to = x[0] >> p.ls[0];
