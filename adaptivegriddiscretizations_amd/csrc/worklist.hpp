@@ -351,6 +351,7 @@ __global__ inline void __launch_bounds__(64) bab_threshold_kernel(int32_t* ctl, 
 }
 
 struct WorklistResult {
+  int64_t seen = 0;  // while passes are queued ahead: visits of those known to have begun
   int64_t passes = 0;      // launches issued
   int64_t niter = 0;       // passes with a non-empty list
   int64_t visits = 0;      // tile visits
@@ -451,6 +452,7 @@ int run_worklist(Workspace& wsr, int32_t ntiles, int32_t grid, int64_t nitermax,
       }
       if (len[begun] >= 0) {
         converged = len[begun] == 0;
+        res.seen += len[begun];
         ++begun;
         idle = 0;
       } else if (++idle > 4096) {
