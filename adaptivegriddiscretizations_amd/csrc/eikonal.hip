@@ -699,9 +699,12 @@ static int region_impl(Workspace& ws, const EikArgs<S>& e, const agd_eikonal_des
                b_done = up(size_t(p.nregions) * kRegionLine * 4), b_marks = up(size_t(ntiles) * 4),
                b_read = up(size_t(ntiles) * 8), b_zero = b_ctl + b_rest + b_done + b_marks + b_read, b_link = up(size_t(ntiles) * 256),
                b_blk = size_t(ntiles) * size_t(rk.tile_bytes);
-  int st = ws.ensure(1, 1, 1);
-  if (!st) st = ws.ensure_region(b_zero + b_link + b_blk);
+  const int st = ws.ensure(1, 1, 1);
   if (st) return st;
+  if (ws.ensure_region(b_zero + b_link + b_blk) != AGD_OK) {
+    (void)hipGetLastError();  // no room: the pass solver needs less
+    return AGD_OK;
+  }
   char* base = static_cast<char*>(ws.region);
   RegionArgs<S> a{};
   a.p = p;
@@ -745,11 +748,11 @@ static int region_impl(Workspace& ws, const EikArgs<S>& e, const agd_eikonal_des
   hipLaunchKernelGGL(rk.solve, dim3(unsigned(p.nregions)), dim3(unsigned(64 * rk.waves)), lds, stream, a);
   AGD_HIP_TRY(hipGetLastError());
   AGD_HIP_TRY(hipEventRecord(ws.ev1, stream));
-  touched = true;
   AGD_HIP_TRY(hipMemcpyAsync(ws.host_counts, a.ctl, kRegionCtl * 4, hipMemcpyDeviceToHost, stream));
   AGD_HIP_TRY(hipStreamSynchronize(stream));
   ws.busy = false;
   const uint32_t* c = reinterpret_cast<const uint32_t*>(ws.host_counts);
+  touched = c[kRegionGo] == 1u;
   if (c[kRegionFinished] != 1u) return AGD_OK;
   taken = true;
   if (stats) {

@@ -312,6 +312,9 @@ __global__ void __launch_bounds__(256) region_setup(RegionArgs<S> a) {
   const S rhs = dom ? a.rhs[n] : inf_v<S>();
   const bool seed = dom && ((a.seeds[n >> 5] >> (n & 31)) & 1u);
   if (seed) a.u[n] = rhs;
+  // (a NaN among the values is for the pass solver, which keeps it: the
+  // minimum and the sort of region_solve pass over it)
+  if (__any(dom && isnan_(seed ? rhs : a.u[n])) && lane == 0) atomicCAS(a.ctl + kRegionGo, 0u, 2u);
   const bool live = dom && !seed;
   const bool trig = dom && (a.activate_all || ((a.trigger[n >> 5] >> (n & 31)) & 1u));
 

@@ -107,3 +107,25 @@ def test_solve_continues_from_given_values():
     u = a['values'].cpu().numpy()
     b = _solve('Riemann3', (37, 21, 30), 'FIM', values=(u + 0.3).astype(np.float32), warmStartAllTiles=True)
     assert np.max(np.abs(b['values'].cpu().numpy() - u)) <= 1e-4 * np.max(np.abs(u))
+
+
+@pytest.mark.parametrize("model,fp64", [('Isotropic2', False), ('Riemann2', True)])
+def test_nan_seed_stays_and_blocks_as_in_the_pass_solver(model, fp64):
+    """A seed of value NaN keeps it, and a cell that reads it is not updated."""
+    rng = np.random.default_rng(4)
+    dims = (40, 33)
+    out = {}
+    for solver in ('FIM', 'AGSI'):
+        h = Eikonal.dictIn({'model': model, 'exportValues': True, 'verbosity': 0, 'solver': solver})
+        h.SetRect([[0, n / 16.] for n in dims], dims=list(dims))
+        h['seeds'] = ((np.array([[4, 5], [30, 20]]) + 0.5) / 16.).astype(np.float32)
+        h['seedValues'] = np.array([0., np.nan])
+        if model == 'Riemann2':
+            h['metric'] = Metrics.Riemann(_metric(np.random.default_rng(5), 2, dims))
+        h['cost'] = np.ones(dims, np.float32)
+        if fp64:
+            h['values_float64'] = True
+        out[solver] = h.Run()['values'].cpu().numpy()
+    u, v = out['FIM'], out['AGSI']
+    assert np.isnan(u[30, 20]) and np.isnan(v[30, 20])
+    assert np.array_equal(np.isnan(u), np.isnan(v)) and np.array_equal(np.isinf(u), np.isinf(v))
