@@ -458,7 +458,7 @@ int agd_scatter_seeds(int32_t scalar, int64_t nseeds, const int64_t* tiled_index
 
 /* Walls (_SetGeometry.py:262-282, _SetArgs.py:124-126): wall cells get
  * rhs = +inf and their seed bit; wall_dist = saturated L1 distance to the
- * walls (computed by `bound` min-plus passes, Kernel_InfConvolution.h),
+ * walls (as `bound` min-plus passes give, Kernel_InfConvolution.h),
  * 255 beyond `bound`.  walls: tiled uint8 mask (padding = 0). */
 int agd_prepare_walls(const agd_eikonal_desc* desc, const uint8_t* walls, int32_t bound,
                       void* rhs, uint32_t* seeds, uint8_t* wall_dist, void* stream);
