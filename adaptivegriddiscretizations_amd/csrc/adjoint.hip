@@ -138,12 +138,17 @@ __global__ void fwd_fill(int64_t N, int nsym, const S* fw, const int32_t* fidx,
 // (_PostProcess.py:143-144): in reverse mode no cell uses them as upwind
 // neighbour, in forward mode they have no upwind neighbour (seeds).
 template <class S>
-__global__ void adj_trigger(int64_t N, const S* u, const int32_t* rowptr, uint32_t* trig) {
+__global__ void __launch_bounds__(256) adj_trigger(int64_t N, const S* u, const int32_t* rowptr, uint32_t* trig) {
   const int64_t y = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (y >= N) return;
-  const S v = u[y];
-  if (rowptr[y + 1] == rowptr[y] && v == v && v != inf_v<S>())
-    atomicOr(trig + (y >> 5), 1u << (y & 31));
+  bool on = false;
+  if (y < N) {
+    const S v = u[y];
+    on = rowptr[y + 1] == rowptr[y] && v == v && v != inf_v<S>();
+  }
+  // (N is a multiple of 64; lanes 0 and 32 each store a word)
+  const uint64_t m = __ballot(on);
+  const int lane = threadIdx.x & 63;
+  if (y < N && (lane & 31) == 0) trig[y >> 5] = uint32_t(m >> lane);
 }
 
 template <class S> struct LinArgs {
@@ -167,13 +172,23 @@ template <class S> __global__ void fill_inf_kernel(int64_t n, S* x) {
 
 template <class S> __device__ inline S init_val(S x) { return x == inf_v<S>() ? S(0) : x; }
 
+// A visit waits for three rounds of loads in a row: the row bounds, the entries
+// of the row, the values of those outside the tile.  The first kRowRegs entries
+// of every row are loaded together (with one entry after the other, each of
+// them two rounds, a pass of 97 x 101 x 89 took 12.9 us and one of 501 x 403 8.9 us;
+// here 9.6 and 7.0).  Tiles of one wave sweep without a barrier, larger ones between two
+// copies of the values with one barrier a sweep.
+constexpr int kRowRegs = 8;
 template <class S, int D, int T0, int T1, int T2>
 __global__ void __launch_bounds__(T0* T1* T2) adj_update(LinArgs<S> a) {
   static_assert((T0 * T1 * T2) % 64 == 0, "tiles are whole waves (pass_begin scans per wave)");
   using TL = Tile<D, T0, T1, T2>;
   constexpr int NI = TL::NI;
   static_assert((NI & (NI - 1)) == 0, "in-tile slots are taken as src & (NI - 1)");
-  __shared__ S l_s[NI];
+  constexpr int K = kRowRegs;
+  __shared__ S l_s[NI > 64 ? 2 * NI : NI];
+  __shared__ uint32_t any_s[NI > 64 ? 2 * (NI / 64) : 1];
+  int turn = 0;
   const int tid = threadIdx.x;
   const PassView pv = pass_begin(a.w);
   const int count = pv.count;
@@ -188,41 +203,72 @@ __global__ void __launch_bounds__(T0* T1* T2) adj_update(LinArgs<S> a) {
     const S dg = a.diag[n_t];
     const S diag = dg == S(0) ? S(1) : dg;
     const int32_t r0 = a.rowptr[n_t], rl = a.rowloc[n_t], r1 = a.rowptr[n_t + 1];
+    int32_t sk[K];
+    S wk[K], out[K];
+#pragma unroll
+    for (int q = 0; q < K; ++q) {
+      const bool in = r0 + q < r1;
+      sk[q] = in ? a.src[r0 + q] : int32_t(n_t);
+      wk[q] = in ? a.wt[r0 + q] : S(0);
+    }
+#pragma unroll
+    for (int q = 0; q < K; ++q) out[q] = (r0 + q >= rl && r0 + q < r1) ? a.lam[sk[q]] : S(0);
     // sources outside the tile: fixed during the visit, summed once
     S sum_out = rhs;
-    for (int32_t j = rl; j < r1; ++j) sum_out += a.wt[j] * init_val(a.lam[a.src[j]]);
-    // in-tile sources: the first K held in registers (a zero weight pads
-    // shorter rows), any further ones re-read at every sweep
-    constexpr int K = 8;
+#pragma unroll
+    for (int q = 0; q < K; ++q)
+      if (r0 + q >= rl && r0 + q < r1) sum_out += wk[q] * init_val(out[q]);
+    for (int32_t j = max(rl, r0 + K); j < r1; ++j) sum_out += a.wt[j] * init_val(a.lam[a.src[j]]);
+    // in-tile sources: slots and weights in registers (a zero weight pads
+    // shorter rows), those after the first K re-read at every sweep
     int slot[K];
-    S wk[K];
 #pragma unroll
     for (int q = 0; q < K; ++q) {
       const bool in = r0 + q < rl;
-      slot[q] = in ? (a.src[r0 + q] & (NI - 1)) : tid;
-      wk[q] = in ? a.wt[r0 + q] : S(0);
+      slot[q] = in ? (sk[q] & (NI - 1)) : tid;
+      wk[q] = in ? wk[q] : S(0);
     }
-    l_s[tid] = init_val(lold);
+    S val = init_val(lold);
+    l_s[tid] = val;
     __syncthreads();
-    for (int it = 0; it < a.niter_i; ++it) {
+    auto sweep = [&](const S* from, S* to) {
+      compiler_fence();
+      S x[K];
+#pragma unroll
+      for (int q = 0; q < K; ++q) x[q] = from[slot[q]];
       S sum = sum_out;
 #pragma unroll
-      for (int q = 0; q < K; ++q) sum += wk[q] * l_s[slot[q]];
-      for (int32_t j = r0 + K; j < rl; ++j) sum += a.wt[j] * l_s[a.src[j] & (NI - 1)];
-      const S nv = sum / diag;
-      __syncthreads();
-      const bool ch = !(nv == l_s[tid]);
-      l_s[tid] = nv;
-      if (!__syncthreads_or(ch)) break;
+      for (int q = 0; q < K; ++q) sum += wk[q] * x[q];
+      for (int32_t j = r0 + K; j < rl; ++j) sum += a.wt[j] * from[a.src[j] & (NI - 1)];
+      val = sum / diag;
+      to[tid] = val;
+      compiler_fence();
+    };
+    // (until a sweep changes nothing: the next would read the same values)
+    if constexpr (NI <= 64) {
+      for (int it = 0; it < a.niter_i; ++it) {
+        const S before = val;
+        sweep(l_s, l_s);
+        if (!__any(!(val == before))) break;
+      }
+    } else {
+      S *from = l_s, *to = l_s + NI;
+      for (int it = 0; it < a.niter_i; ++it) {
+        const S before = val;
+        sweep(from, to);
+        if (!tile_any<NI>(!(val == before), any_s, turn)) break;
+        S* const t = from;
+        from = to;
+        to = t;
+      }
     }
-    const S val = l_s[tid];
     a.lam[n_t] = val;
     const S tol = abs_(val) * a.rtol + a.atol;
-    const bool changed = abs_(val - lold) > tol;
-    const bool any = __syncthreads_or(changed);
-    if (any && tid < 2 * D + 1) {
-      const int nb = (tid == 2 * D) ? n_o : tile_neighbor<D>(xo, tid >> 1, 2 * (tid & 1) - 1, a.g);
-      if (nb >= 0) enqueue(nb, tag, a.w.stamp, pv.list_out, pv.count_out);
+    const bool any = tile_any<NI>(abs_(val - lold) > tol, any_s, turn);
+    if (tid < 64) {
+      int nb = -1;
+      if (tid < 2 * D + 1) nb = (tid == 2 * D) ? n_o : tile_neighbor<D>(xo, tid >> 1, 2 * (tid & 1) - 1, a.g);
+      enqueue_wave(any && nb >= 0, nb, nb, tag, a.w.stamp, pv.list_out, pv.count_out);
     }
     __syncthreads();
   }
@@ -235,8 +281,11 @@ __global__ void __launch_bounds__(64) adj_init_list(const uint32_t* trigger, int
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   bool on = false;
   if (t < ntiles) {
-    const int64_t b0 = int64_t(t) * NI, b1 = b0 + NI;
-    for (int64_t b = b0; b < b1 && !on; ++b) on = (trigger[b >> 5] >> (b & 31)) & 1u;
+    static_assert(NI % 32 == 0, "a tile's trigger bits are whole words");
+    uint32_t bits = 0;
+#pragma unroll
+    for (int i = 0; i < NI / 32; ++i) bits |= trigger[int64_t(t) * (NI / 32) + i];
+    on = bits != 0;
   }
   const int shard = blockIdx.x % kShards;
   enqueue_wave(on, on ? t : 0, t, 0, stamp, lists + int64_t(shard) * shard_cap,
@@ -299,7 +348,7 @@ static int linear_impl(bool forward, const agd_eikonal_desc* d, const S* values,
   const dim3 grid(unsigned(ceil_div(N, 256))), block(256);
 
   // ---- 1. the system's rows (reverse: transposed flow graph), in the
-  // workspace: [deg, trig (cleared)], rowptr, rowloc, the scan's own
+  // workspace: deg (cleared), trig, rowptr, rowloc, the scan's own
   WorkspaceLease lease;
   Workspace& ws = *lease;
   size_t tmp_bytes = 0;
@@ -315,7 +364,7 @@ static int linear_impl(bool forward, const agd_eikonal_desc* d, const S* values,
   int32_t* const rowptr = reinterpret_cast<int32_t*>(base + b_deg + b_trig);
   int32_t* const rowloc = reinterpret_cast<int32_t*>(base + 2 * b_deg + b_trig);
   void* const tmp = base + 2 * b_deg + b_trig + b_loc;
-  fill_i32(deg, int64_t((b_deg + b_trig) / 4), 0, stream);
+  fill_i32(deg, N + 1, 0, stream);
   if (forward)
     hipLaunchKernelGGL(fwd_count<S>, grid, block, 0, stream, N, nsym, fw, fidx, deg);
   else

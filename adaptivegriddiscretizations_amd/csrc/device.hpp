@@ -64,6 +64,25 @@ template <class T> __device__ inline void st32(T* base, uint32_t idx, T v) {
   *reinterpret_cast<T*>(reinterpret_cast<char*>(base) + idx * uint32_t(sizeof(T))) = v;
 }
 
+// Tile-wide "any" of a workgroup of NI lanes: a ballot for one wave; otherwise
+// one barrier, which also ends the LDS accesses before it (flags alternates
+// between two sets of NI / 64).
+template <int NI> __device__ inline bool tile_any(bool p, uint32_t* flags, int& turn) {
+  if constexpr (NI <= 64) {
+    return __ballot(p) != 0;
+  } else {
+    uint32_t* const f = flags + turn * (NI / 64);
+    turn ^= 1;
+    const bool wave = __ballot(p) != 0;
+    if ((threadIdx.x & 63) == 0) f[threadIdx.x >> 6] = wave;
+    __syncthreads();
+    uint32_t any = 0;
+#pragma unroll
+    for (int w = 0; w < NI / 64; ++w) any |= f[w];
+    return any != 0;
+  }
+}
+
 // ------------------------------------------------------------------ models
 template <int MODEL, int D> struct ModelTraits {
   static constexpr int SYMDIM = D * (D + 1) / 2;

@@ -231,24 +231,6 @@ template <int NI> __device__ inline bool block_any(bool p) {
   }
 }
 
-// The same with one barrier, which also ends the LDS accesses before it: flags
-// alternates between two sets of NI / 64 flags.
-template <int NI> __device__ inline bool tile_any(bool p, uint32_t* flags, int& turn) {
-  if constexpr (NI <= 64) {
-    return __ballot(p) != 0;
-  } else {
-    uint32_t* const f = flags + turn * (NI / 64);
-    turn ^= 1;
-    const bool wave = __ballot(p) != 0;
-    if ((threadIdx.x & 63) == 0) f[threadIdx.x >> 6] = wave;
-    __syncthreads();
-    uint32_t any = 0;
-#pragma unroll
-    for (int w = 0; w < NI / 64; ++w) any |= f[w];
-    return any != 0;
-  }
-}
-
 // Block-wide minimum (the same value in every thread).
 template <int NI, class S> __device__ inline S block_min(S v) {
 #pragma unroll
