@@ -10,11 +10,11 @@
 //
 // MI355X formulation:
 //  1. transpose the flow graph into CSR rows indexed by the upwind cell y:
-//     in-degree count (atomics), exclusive scan (hipCUB), scatter (atomic
-//     cursors), then each row sorted by source index so the summation order,
-//     hence the FP32 result, is deterministic;
-//  2. each row stably partitioned into the sources inside the row's tile,
-//     then those outside (rowloc marks the split);
+//     in-degree count (atomics, whose results are the entries' places),
+//     exclusive scan (hipCUB), scatter;
+//  2. each row ordered by source index, those inside the row's tile first
+//     (rowloc marks the split), so that the summation order, hence the FP32
+//     result, is deterministic;
 //  3. tile Gauss-Seidel on the transposed system with the same device
 //     worklist as the eikonal solver (AGSI activation, as the reference's
 //     SolveLinear switches FIM to AGSI, _PostProcess.py:117-118).  The tile's
@@ -26,6 +26,7 @@
 #include <hipcub/hipcub.hpp>
 
 #include <cstring>
+#include <type_traits>
 #include <vector>
 
 #include "common.hpp"
@@ -34,53 +35,125 @@
 
 namespace agd {
 
+// The workgroups of an XCD (every eighth) take one stretch of the cells: their
+// entries fall into rows of the same stretch, whose cache lines the XCD's L2
+// then fills by itself.
+__device__ inline uint32_t xcd_block() {
+  const uint32_t n = gridDim.x, x = blockIdx.x & 7, base = n >> 3, rest = n & 7;
+  return x * base + min(x, rest) + (blockIdx.x >> 3);
+}
+
+// In-degrees, and the place of every entry in its (unordered) row.  (The rate
+// of the atomics bounds it: several in flight per lane, or a stretch of the
+// cells per XCD, do not make it faster.)
 template <class S>
-__global__ void adj_count(int64_t N, int nsym, const S* fw, const int32_t* fidx, int32_t* deg) {
+__global__ void adj_count(int64_t N, int nsym, const S* fw, const int32_t* fidx, int32_t* deg, int32_t* place) {
   const int64_t x = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (x >= N) return;
   for (int k = 0; k < nsym; ++k) {
     const int32_t y = fidx[k * N + x];
-    if (fw[k * N + x] != S(0) && y != INT32_MAX) atomicAdd(deg + y, 1);
+    if (fw[k * N + x] != S(0) && y != INT32_MAX) place[k * N + x] = atomicAdd(deg + y, 1);
   }
 }
 
+template <class S> struct RowEntry {
+  int32_t src;
+  S wt;
+};
+
+// Source and weight in one store, as the rows of a wave's cells are scattered;
+// the loads of kEdges neighbours are in flight together.
+constexpr int kEdges = 6;
 template <class S>
-__global__ void adj_fill(int64_t N, int nsym, const S* fw, const int32_t* fidx, int32_t* cursor,
-                         int32_t* src, S* wt) {
-  const int64_t x = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+__global__ void __launch_bounds__(256) adj_fill(int64_t N, int nsym, const S* __restrict__ fw,
+                                                const int32_t* __restrict__ fidx,
+                                                const int32_t* __restrict__ rowptr,
+                                                const int32_t* __restrict__ place, RowEntry<S>* __restrict__ rows) {
+  const int64_t x = int64_t(xcd_block()) * blockDim.x + threadIdx.x;
   if (x >= N) return;
-  for (int k = 0; k < nsym; ++k) {
-    const int32_t y = fidx[k * N + x];
-    const S w = fw[k * N + x];
-    if (w != S(0) && y != INT32_MAX) {
-      const int32_t p = atomicAdd(cursor + y, 1);
-      src[p] = int32_t(x);
-      wt[p] = w;
+  for (int k0 = 0; k0 < nsym; k0 += kEdges) {
+    int32_t y[kEdges], p[kEdges];
+    S w[kEdges];
+#pragma unroll
+    for (int q = 0; q < kEdges; ++q) {
+      const int64_t i = int64_t(min(k0 + q, nsym - 1)) * N + x;
+      y[q] = fidx[i];
+      w[q] = fw[i];
+      p[q] = place[i];
+      if (!(k0 + q < nsym && w[q] != S(0))) y[q] = INT32_MAX;
     }
+#pragma unroll
+    for (int q = 0; q < kEdges; ++q)
+      if (y[q] != INT32_MAX) p[q] += rowptr[y[q]];
+#pragma unroll
+    for (int q = 0; q < kEdges; ++q)
+      if (y[q] != INT32_MAX) rows[p[q]] = RowEntry<S>{int32_t(x), w[q]};
   }
 }
 
-// Sort each row by source index (rows hold a handful of entries).
+// Every row in its final order: the sources inside the row's own tile (of ni
+// cells) by index, then the others by index; rowloc[y] = end of the in-tile
+// part.  An entry goes to its rank, the number of smaller keys (a
+// source twice in a row, on a short periodic axis, keeps its place); rows of up to
+// 16 entries are ranked in registers.  (97 x 101 x 89: filling with atomics, insertion
+// sort and partition in memory took 87, 84 and 48 us; filling takes 35 us, this 37.)
 template <class S>
-__global__ void adj_sort_rows(int64_t N, const int32_t* rowptr, int32_t* src, S* wt) {
+__global__ void __launch_bounds__(256) adj_order_rows(int64_t N, int ni, const int32_t* rowptr,
+                                                      const RowEntry<S>* rows, int32_t* src, S* wt,
+                                                      int32_t* rowloc) {
   const int64_t y = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (y >= N) return;
-  const int32_t r0 = rowptr[y], r1 = rowptr[y + 1];
-  for (int32_t i = r0 + 1; i < r1; ++i) {
-    const int32_t s = src[i];
-    const S w = wt[i];
-    int32_t j = i - 1;
-    while (j >= r0 && src[j] > s) {
-      src[j + 1] = src[j];
-      wt[j + 1] = wt[j];
-      --j;
+  const int32_t r0 = rowptr[y], n = rowptr[y + 1] - r0;
+  const int32_t tile = int32_t(y / ni);
+  rows += r0;
+  src += r0;
+  wt += r0;
+  auto key = [&](int32_t s) { return uint32_t(s) | (s / ni != tile ? 0x80000000u : 0u); };
+  int in = 0;
+  auto ranked = [&](auto regs) {
+    constexpr int R = decltype(regs)::value;
+    uint32_t k[R];
+    S w[R];
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const RowEntry<S> e = i < n ? rows[i] : RowEntry<S>{0, S(0)};
+      k[i] = i < n ? key(e.src) : 0xffffffffu;
+      w[i] = e.wt;
     }
-    src[j + 1] = s;
-    wt[j + 1] = w;
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      int rank = 0;
+#pragma unroll
+      for (int j = 0; j < R; ++j) rank += j < i ? k[j] <= k[i] : (j > i && k[j] < k[i]);
+      if (i < n) {
+        src[rank] = int32_t(k[i] & 0x7fffffffu);
+        wt[rank] = w[i];
+        in += !(k[i] >> 31);
+      }
+    }
+  };
+  if (n <= 6) {
+    ranked(std::integral_constant<int, 6>{});
+  } else if (n <= 16) {
+    ranked(std::integral_constant<int, 16>{});
+  } else {
+    for (int i = 0; i < n; ++i) {
+      const RowEntry<S> e = rows[i];
+      const uint32_t ke = key(e.src);
+      int rank = 0;
+      for (int j = 0; j < n; ++j) {
+        const uint32_t kj = key(rows[j].src);
+        rank += j < i ? kj <= ke : (j > i && kj < ke);
+      }
+      src[rank] = e.src;
+      wt[rank] = e.wt;
+      in += !(ke >> 31);
+    }
   }
+  rowloc[y] = r0 + in;
 }
 
-// Stable partition of every row: sources in the row's own tile (of NI
+// Forward rows, in stencil order.  Stable partition of every row: sources in the row's own tile (of NI
 // cells) first, then the others; rowloc[y] = end of the in-tile part.
 template <class S>
 __global__ void lin_partition_rows(int64_t N, int ni, const int32_t* rowptr, int32_t* src, S* wt,
@@ -173,19 +246,19 @@ template <class S> __global__ void fill_inf_kernel(int64_t n, S* x) {
 template <class S> __device__ inline S init_val(S x) { return x == inf_v<S>() ? S(0) : x; }
 
 // A visit waits for three rounds of loads in a row: the row bounds, the entries
-// of the row, the values of those outside the tile.  The first kRowRegs entries
-// of every row are loaded together (with one entry after the other, each of
-// them two rounds, a pass of 97 x 101 x 89 took 12.9 us and one of 501 x 403 8.9 us;
-// here 9.6 and 7.0).  Tiles of one wave sweep without a barrier, larger ones between two
-// copies of the values with one barrier a sweep.
-constexpr int kRowRegs = 8;
+// of the row, the values of those outside the tile.  The first K entries of
+// every row are loaded together (with one entry after the other, each of them
+// two rounds, a pass of 97 x 101 x 89 took 12.9 us and one of 501 x 403 8.9 us; here 9.6
+// and 7.0; 16 entries at once gain nothing more).  Tiles of one wave sweep
+// without a barrier, larger ones between two copies of the values with one
+// barrier a sweep.
 template <class S, int D, int T0, int T1, int T2>
 __global__ void __launch_bounds__(T0* T1* T2) adj_update(LinArgs<S> a) {
   static_assert((T0 * T1 * T2) % 64 == 0, "tiles are whole waves (pass_begin scans per wave)");
   using TL = Tile<D, T0, T1, T2>;
   constexpr int NI = TL::NI;
   static_assert((NI & (NI - 1)) == 0, "in-tile slots are taken as src & (NI - 1)");
-  constexpr int K = kRowRegs;
+  constexpr int K = 8;
   __shared__ S l_s[NI > 64 ? 2 * NI : NI];
   __shared__ uint32_t any_s[NI > 64 ? 2 * (NI / 64) : 1];
   int turn = 0;
@@ -348,44 +421,56 @@ static int linear_impl(bool forward, const agd_eikonal_desc* d, const S* values,
   const dim3 grid(unsigned(ceil_div(N, 256))), block(256);
 
   // ---- 1. the system's rows (reverse: transposed flow graph), in the
-  // workspace: deg (cleared), trig, rowptr, rowloc, the scan's own
+  // workspace: deg (cleared), trig, rowptr, rowloc, place, the scan's own;
+  // src, wt, and in reverse mode the rows before they are ordered
   WorkspaceLease lease;
   Workspace& ws = *lease;
   size_t tmp_bytes = 0;
   AGD_HIP_TRY(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp_bytes, static_cast<int32_t*>(nullptr),
                                                static_cast<int32_t*>(nullptr), int(N + 1), stream));
   auto up = [](size_t b) { return (b + 255) & ~size_t(255); };
-  const size_t b_deg = up(size_t(N + 1) * 4), b_trig = up(size_t(ceil_div(N, 32)) * 4), b_loc = up(size_t(N) * 4);
-  if (int st = ws.ensure_scratch(2 * b_deg + b_trig + b_loc + tmp_bytes)) return st;
+  const int64_t most = int64_t(nsym) * N;  // entries
+  const size_t b_deg = up(size_t(N + 1) * 4), b_trig = up(size_t(ceil_div(N, 32)) * 4), b_loc = up(size_t(N) * 4),
+               b_place = forward ? 0 : up(size_t(most) * 4);
+  if (int st = ws.ensure_scratch(2 * b_deg + b_trig + b_loc + b_place + tmp_bytes)) return st;
   ws.busy = true;
   char* const base = static_cast<char*>(ws.scratch);
   int32_t* const deg = reinterpret_cast<int32_t*>(base);
   uint32_t* const trig = reinterpret_cast<uint32_t*>(base + b_deg);
   int32_t* const rowptr = reinterpret_cast<int32_t*>(base + b_deg + b_trig);
   int32_t* const rowloc = reinterpret_cast<int32_t*>(base + 2 * b_deg + b_trig);
-  void* const tmp = base + 2 * b_deg + b_trig + b_loc;
+  int32_t* const place = reinterpret_cast<int32_t*>(base + 2 * b_deg + b_trig + b_loc);
+  void* const tmp = base + 2 * b_deg + b_trig + b_loc + b_place;
   fill_i32(deg, N + 1, 0, stream);
   if (forward)
     hipLaunchKernelGGL(fwd_count<S>, grid, block, 0, stream, N, nsym, fw, fidx, deg);
   else
-    hipLaunchKernelGGL(adj_count<S>, grid, block, 0, stream, N, nsym, fw, fidx, deg);
+    hipLaunchKernelGGL(adj_count<S>, grid, block, 0, stream, N, nsym, fw, fidx, deg, place);
   AGD_HIP_TRY(hipcub::DeviceScan::ExclusiveSum(tmp, tmp_bytes, deg, rowptr, int(N + 1), stream));
-  int32_t nnz = 0;
-  AGD_HIP_TRY(hipMemcpyAsync(&nnz, rowptr + N, sizeof(int32_t), hipMemcpyDeviceToHost, stream));
-  AGD_HIP_TRY(hipStreamSynchronize(stream));
-  const size_t b_src = up(size_t(std::max<int64_t>(nnz, 1)) * 4);
-  if (int st = ws.ensure_region(b_src + size_t(std::max<int64_t>(nnz, 1)) * sizeof(S))) return st;
+  // Room for as many entries as there can be where that is little; else for
+  // their number, read back (the call waits 25 us for it).
+  auto b_rows = [&](int64_t n) {
+    return up(size_t(n) * 4) + up(size_t(n) * sizeof(S)) + (forward ? 0 : up(size_t(n) * sizeof(RowEntry<S>)));
+  };
+  int64_t room = most;
+  if (b_rows(most) > (size_t(256) << 20)) {
+    int32_t nnz = 0;
+    AGD_HIP_TRY(hipMemcpyAsync(&nnz, rowptr + N, sizeof(int32_t), hipMemcpyDeviceToHost, stream));
+    AGD_HIP_TRY(hipStreamSynchronize(stream));
+    room = std::max<int64_t>(nnz, 1);
+  }
+  if (int st = ws.ensure_region(b_rows(room))) return st;
   int32_t* const src = static_cast<int32_t*>(ws.region);
-  S* const wt = reinterpret_cast<S*>(static_cast<char*>(ws.region) + b_src);
+  S* const wt = reinterpret_cast<S*>(static_cast<char*>(ws.region) + up(size_t(room) * 4));
   if (forward) {
     hipLaunchKernelGGL(fwd_fill<S>, grid, block, 0, stream, N, nsym, fw, fidx, rowptr, src, wt);
+    hipLaunchKernelGGL(lin_partition_rows<S>, grid, block, 0, stream, N, ls.ni, rowptr, src, wt, rowloc);
   } else {
-    AGD_HIP_TRY(hipMemcpyAsync(deg, rowptr, (N + 1) * sizeof(int32_t), hipMemcpyDeviceToDevice,
-                               stream));
-    hipLaunchKernelGGL(adj_fill<S>, grid, block, 0, stream, N, nsym, fw, fidx, deg, src, wt);
-    hipLaunchKernelGGL(adj_sort_rows<S>, grid, block, 0, stream, N, rowptr, src, wt);
+    auto* const rows =
+        reinterpret_cast<RowEntry<S>*>(reinterpret_cast<char*>(wt) + up(size_t(room) * sizeof(S)));
+    hipLaunchKernelGGL(adj_fill<S>, grid, block, 0, stream, N, nsym, fw, fidx, rowptr, place, rows);
+    hipLaunchKernelGGL(adj_order_rows<S>, grid, block, 0, stream, N, ls.ni, rowptr, rows, src, wt, rowloc);
   }
-  hipLaunchKernelGGL(lin_partition_rows<S>, grid, block, 0, stream, N, ls.ni, rowptr, src, wt, rowloc);
   hipLaunchKernelGGL(adj_trigger<S>, grid, block, 0, stream, N, values, rowptr, trig);
   AGD_HIP_TRY(hipGetLastError());
 
