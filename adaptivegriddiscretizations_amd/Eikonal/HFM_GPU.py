@@ -791,7 +791,7 @@ class Interface:
         return io
 
     def solver_handle(self):
-        """The solver handle (worklist workspace, cached pass graph) of this
+        """The solver handle (worklist workspace) of this
         run, bound to its stream; created on first use."""
         h = getattr(self, '_solver_handle', None)
         if h is None:

@@ -87,7 +87,7 @@ class Batch:
             self.inst[i].atol = it.atol
             self.inst[i].rtol = it.rtol
         self.stream = stream_handle()
-        self.solver = _lib.Solver(self.stream)  # worklist workspace, cached pass graph
+        self.solver = _lib.Solver(self.stream)  # worklist workspace
         self.ncells = int(sum(int(np.prod(it.shape)) for it in self.ifaces))
 
     def _cat_bits(self, name):
