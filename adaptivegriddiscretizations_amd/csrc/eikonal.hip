@@ -699,6 +699,13 @@ static int region_impl(Workspace& ws, const EikArgs<S>& e, const agd_eikonal_des
   const RegionKernels<S> rk = region_lookup<S>(d->model, d->ndim);
   if (!rk.solve || hipGetDevice(&dev) != hipSuccess || dev >= kMaxDevices || !region_plan(d, rk.box, rk.waves, rk.lds, p))
     return AGD_OK;
+  // Riemannian volumes of more tiles than two for each of 16 waves on 256 compute
+  // units: the passes, which read stored stencils by then, keep more tiles in
+  // flight.  (60^3, 3375 tiles: 0.86 ms a call in one launch, 1.06 in passes; 90^3, 12167:
+  // 1.51, 1.41; 120 x 110 x 100: 2.00, 1.64; 170 x 160 x 170: 4.82, 2.86.)
+  if (std::is_same<S, float>::value && d->model == AGD_RIEMANN && d->ndim == 3 &&
+      int64_t(p.ntl[0]) * p.ntl[1] * p.ntl[2] > 8192)
+    return AGD_OK;
   std::unique_lock<std::mutex> lock(g_region_mutex[dev], std::try_to_lock);
   if (!lock.owns_lock()) return AGD_OK;
   const int64_t ntiles = int64_t(p.nregions) * p.ntot;
